@@ -42,6 +42,12 @@ namespace {
 constexpr uint32_t kMaxIterationsCap = 1u << 24;
 constexpr uint32_t kMaxCheckEvery = 1u << 16;
 
+// Iteration caps up to which a refinement may be one resident launch (up to
+// ~30 us per iteration), and the 64-bit words its workgroups publish (six
+// for each of at most 256).
+constexpr uint32_t kResidentCap = 16384;
+constexpr uint32_t kResidentWords = 6 * 256;
+
 // One validator for every way a configuration enters the simulation
 // (creation, set_config, snapshot load).
 void validate_config(const FluidConfig& c) {
@@ -513,6 +519,50 @@ SolveStats FluidSim::solveWith(int prec) {
     return solveOnce(prec, cfg_.maxIterations);
 }
 
+// One refinement by the resident PCG: x64 += e with A e = (float) r64, then
+// r64 = b - A x64 and its squared norm, with one wait for the device.
+FluidSim::ResidentEnd FluidSim::residentRefinement(uint32_t na, const ns::ResidentShape& shape, bool mic,
+                                                   const double* r64, double thr2, uint32_t limit) {
+    int dev = 0;
+    FLIP2_HIP(hipGetDevice(&dev));
+    const uint64_t last = (uint64_t)residentNumber_ + 2u * (uint64_t)limit + 4u;
+    if (residentNumber_ == 0 || last > 0xffffffffull) {
+        ns::launch_fill_f64(words_.devPtr(), kResidentWords, 0.0, stream_);
+        ns::launch_fill_f64(scal_.devPtr() + 8, 2, 0.0, stream_);
+        residentNumber_ = 1;
+    }
+    // scal[2]: the true residual's norm; scal[8..9]: the kernel's result
+    double* const out = scal_.devPtr() + 2;
+    ns::CgResident c{};
+    c.coef = coef_.devPtr();
+    c.nbrSlot = nbrSlot_.devPtr();
+    c.precon = mic ? precon_.devPtr() : nullptr;
+    c.r64 = r64;
+    c.x64 = x64_.devPtr();
+    c.faces = faces_.devPtr();
+    c.words = reinterpret_cast<uint64_t*>(words_.devPtr());
+    c.result = reinterpret_cast<uint32_t*>(scal_.devPtr() + 8);
+    c.na = na;
+    c.groups = shape.groups;
+    c.limit = limit;
+    c.polls = residentPolls_;
+    c.number = residentNumber_;
+    c.thr2 = thr2;
+    residentNumber_ += 2u * limit + 2u;
+    double* host = pinnedHistory(8);
+    {
+        std::lock_guard<std::mutex> turn(ns::resident_mutex(dev));
+        ns::launch_pcg_resident(c, shape, mic, stream_);
+        ns::launch_true_residual(na, b64_.devPtr(), x64_.devPtr(), coef_.devPtr(), nbrSlot_.devPtr(), r64_.devPtr(),
+                                 reduce(), out, stream_);
+        FLIP2_HIP(hipMemcpyAsync(host, out, 8 * sizeof(double), hipMemcpyDeviceToHost, stream_));
+        synchronize();
+    }
+    uint32_t res[4];
+    std::memcpy(res, host + 6, sizeof(res));
+    return ResidentEnd{host[0], res[0], res[1] == c.number};
+}
+
 SolveStats FluidSim::solveOnce(int prec, uint32_t capIn) {
     SolveStats st;
     const auto t0 = std::chrono::steady_clock::now();
@@ -536,8 +586,6 @@ SolveStats FluidSim::solveOnce(int prec, uint32_t capIn) {
         stats_ = st;
         return st;
     }
-    FLIP2_HIP(hipMemcpyAsync(r64_.devPtr(), b64_.devPtr(), (size_t)cells * sizeof(double), hipMemcpyDeviceToDevice,
-                             stream_));
     FLIP2_REQUIRE(prec != kPrecLearned || learned_, kErrState, "no learned preconditioner installed");
     learnedFresh_ = true;
     if (prec == kPrecMIC0) ns::launch_mic_factor(na, coef_.devPtr(), precon_.devPtr(), stream_);
@@ -545,6 +593,25 @@ SolveStats FluidSim::solveOnce(int prec, uint32_t capIn) {
         ns::launch_mic_factor(na, coef_.devPtr(), precon_.devPtr(), stream_, false);
     const bool jac = prec == kPrecJacobi;
     const bool flex = prec == kPrecLearned;
+    const uint32_t cap = std::min(capIn, cfg_.maxIterations);
+    // Where the slots fit the chip at once, a refinement's whole PCG is one
+    // launch; not with residual capture (it takes r between iterations) or
+    // when a timer is asked for the two-kernel form's launches by name, and
+    // only for caps that end a launch in a fraction of a second.
+    const KernelTimer* timer = KernelTimer::current();
+    const bool perIteration = capture_ || (timer && timer->asksFor("cg_"));
+    const ns::ResidentShape shape = !flex && !perIteration && residentOk_ && cap <= kResidentCap
+                                        ? ns::resident_shape(na, !jac)
+                                        : ns::ResidentShape{0, 0};
+    const bool resident = shape.groups > 0;
+    if (resident) {
+        const size_t want = ns::resident_face_floats(na);
+        if (faces_.size() < want) faces_.resizeAsync((uint32_t)ns::resident_face_floats(slotCapacity_), stream_);
+        if (words_.size() < kResidentWords) words_.resizeAsync(kResidentWords, stream_), residentNumber_ = 0;
+    } else {
+        FLIP2_HIP(hipMemcpyAsync(r64_.devPtr(), b64_.devPtr(), (size_t)cells * sizeof(double),
+                                 hipMemcpyDeviceToDevice, stream_));
+    }
     // Flexible CG: direction of inner iteration j in ring slot j % slots
     // (one more slot than directions kept, so a new direction never
     // overwrites one it is orthogonalised against).
@@ -568,7 +635,6 @@ SolveStats FluidSim::solveOnce(int prec, uint32_t capIn) {
     };
     double rel = 1.0;
     uint32_t total = 0;
-    const uint32_t cap = std::min(capIn, cfg_.maxIterations);
     const uint32_t every = std::max(1u, flex ? cfg_.learnedCheckEvery : cfg_.checkEvery);
     double* H = hist_.devPtr();
     // Flexible CG does not restart at a refinement: the recursive residual is
@@ -586,6 +652,24 @@ SolveStats FluidSim::solveOnce(int prec, uint32_t capIn) {
         // directions across refinements and took more iterations with 2e-6).
         const double innerTol = std::max(0.5 * cfg_.tolerance / rel, flex ? 2e-5 : 2e-6);
         const double ref = rel * st.bNorm;  // norm of the FP32 right-hand side of this refinement
+        if (resident) {
+            const double thr = innerTol * ref;
+            const double* r64 = refine == 0 ? b64_.devPtr() : r64_.devPtr();
+            ResidentEnd end = residentRefinement(na, shape, !jac, r64, thr * thr, cap - total);
+            if (end.failed) {  // x64 is not usable: solve again without it
+                residentOk_ = false;
+                return solveOnce(prec, capIn);
+            }
+            total += end.iterations;
+            rel = std::sqrt(std::max(end.rr, 0.0)) / st.bNorm;
+            st.refinements = refine + 1;
+            if (rel <= cfg_.tolerance) {
+                st.converged = true;
+                break;
+            }
+            if (!(rel == rel)) break;
+            continue;
+        }
         if (!flex) {
             // Jacobi / MIC(0): two kernels per iteration (direction + matvec,
             // update + preconditioner), p alternating between two buffers;

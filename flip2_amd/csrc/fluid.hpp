@@ -142,6 +142,11 @@ public:
         capture_ = std::move(fn);
     }
 
+    // Reads that a wait between the resident PCG's workgroups may take before
+    // it is given up (the solve then runs again in the two-kernel form).
+    void setResidentPolls(uint32_t polls) { residentPolls_ = polls; }
+    bool residentUsable() const { return residentOk_; }
+
     const SolveStats& lastSolve() const { return stats_; }
     uint32_t numParticles() const { return n_; }
     uint32_t numActive() const { return numActive_; }
@@ -225,6 +230,20 @@ private:
     size_t histPinnedDoubles_ = 0;
     hipEvent_t histEvent_[2] = {nullptr, nullptr};
     double* pinnedHistory(size_t doubles);
+    // The resident PCG (ns::launch_pcg_resident): its faces and published
+    // words, the number of its next sum, and whether it may be used (a wait
+    // between its workgroups ran out once: another process shares the GPU).
+    DeviceVec<float> faces_{dm_};
+    DeviceVec<double> words_{dm_};
+    struct ResidentEnd {
+        double rr;
+        uint32_t iterations;
+        bool failed;
+    };
+    ResidentEnd residentRefinement(uint32_t na, const ns::ResidentShape& shape, bool mic, const double* r64,
+                                   double thr2, uint32_t limit);
+    uint32_t residentNumber_ = 0, residentPolls_ = ns::kResidentPolls;
+    bool residentOk_ = true;
     DeviceVec<uint32_t> total_{dm_};
     DeviceVec<uint8_t> ws_{dm_};
     uint32_t slotCapacity_ = 0;

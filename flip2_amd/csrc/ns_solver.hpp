@@ -3,6 +3,8 @@
 
 #include "common.hpp"
 
+#include <mutex>
+
 namespace flip2 {
 namespace ns {
 
@@ -107,6 +109,40 @@ void launch_cg_update_precond(const CgFused& c, uint32_t it, bool init, bool mic
 // history rz, rr of entry `it` from the last update's partials (the values
 // the next matvec would record), for a check at the end of a batch
 void launch_cg_history(const CgFused& c, uint32_t it, hipStream_t s);
+// The whole inner PCG of a refinement in one launch, its vectors resident in
+// registers and LDS (pcg_resident.hip): solves A e = (float) r64 until
+// rr <= thr2 (or rr is not a number) or `limit` iterations, then x64 += e.
+// result (device): [0] iterations; [1] is set to `number` if a wait between
+// the workgroups ran out (x64 is then not usable).
+constexpr int kResidentMaxWaves = 11;
+constexpr uint32_t kResidentPolls = 1u << 18;  // a wait's reads before it is given up (~0.2 s)
+struct CgResident {
+    const uint16_t* coef;
+    const int32_t* nbrSlot;
+    const float* precon;  // MIC(0) factors (null for Jacobi)
+    const double* r64;
+    double* x64;
+    float* faces;     // resident_face_floats(na)
+    uint64_t* words;  // 6 per workgroup, zero before the first launch
+    uint32_t* result;
+    uint32_t na;
+    uint32_t groups;
+    uint32_t limit;
+    uint32_t polls;   // reads of a wait between workgroups before it is given up
+    uint32_t number;  // of the first sum: larger by 2 limit + 2 than the previous launch's on these words
+    double thr2;
+};
+// Workgroups and waves per workgroup for na slots; no groups where they do
+// not fit the chip at once.
+struct ResidentShape {
+    uint32_t groups, waves;
+};
+ResidentShape resident_shape(uint32_t na, bool mic);
+size_t resident_face_floats(uint32_t na);
+// Held from a resident launch until its end: two of them at once could each
+// hold CUs that the other waits for.
+std::mutex& resident_mutex(int device);
+void launch_pcg_resident(const CgResident& c, const ResidentShape& shape, bool mic, hipStream_t s);
 void launch_accumulate(uint32_t numActive, const float* e, double* x64, const uint16_t* coef, hipStream_t s);
 void launch_true_residual(uint32_t numActive, const double* b64, const double* x64, const uint16_t* coef,
                           const int32_t* nbrSlot, double* r64, Reduce red, double* out, hipStream_t s);

@@ -31,6 +31,11 @@ public:
     // around a launch cost the stream a few microseconds, so a timed run of
     // many short launches samples them.
     void setSampleEvery(uint32_t every) { every_ = every ? every : 1u; seen_.clear(); }
+    // Whether the filter names a kernel whose name starts with `prefix`.
+    bool asksFor(const std::string& prefix) const {
+        const auto at = filter_.lower_bound(prefix);
+        return at != filter_.end() && at->compare(0, prefix.size(), prefix) == 0;
+    }
     // Whether the next launch named `name` is recorded (counts it).
     bool wants(const char* name);
     // Record the start / stop event of one launch named `name` on stream s.
