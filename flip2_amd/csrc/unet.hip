@@ -637,17 +637,18 @@ void UNet::forward(hipStream_t s, bool keepActivations) {
                         scale_.devPtr(), out_.devPtr(), (long long)n_ * n_ * n_, 16, s);
 }
 
-// dY: gradient w.r.t. this layer's (post-ReLU) output Y; turned into the
-// pre-activation gradient in place; weight/bias gradients accumulated; dX
+// dY: gradient w.r.t. this layer's (post-ReLU) output Y; weight/bias gradients accumulated; dX
 // (if not null) receives the gradient w.r.t. the layer input X.
-void UNet::convBackward(int layer, float* dY, const uint16_t* Y, const uint16_t* X, float* dX, hipStream_t s) {
+void UNet::convBackward(int layer, const float* dY, const uint16_t* Y, const uint16_t* X, float* dX, hipStream_t s) {
     const UNetLayer& L = layers_[layer];
     const int n = L.level == 0 ? n_ : (L.level == 1 ? n1_ : n2_);
     const long long nvox = (long long)n * n * n;
     if (dPb_.size() < (uint32_t)(nvox * L.cout)) dPb_.resizeAsync((uint32_t)(nvox * L.cout), s);
     if (WT_.size() < (uint32_t)(27 * L.cin * L.cout)) WT_.resizeAsync((uint32_t)(27 * L.cin * L.cout), s);
-    nn::launch_relu_mask_bf16(dY, Y, dPb_.devPtr(), nvox * L.cout, s);
-    nn::launch_conv3_wgrad(dPb_.devPtr(), dY, X, grad_.devPtr() + L.w, grad_.devPtr() + L.b, n, L.cin, L.cout, s);
+    const size_t part = nn::conv3_wgrad_part_floats(n, L.cin, L.cout);
+    if (wgradPart_.size() < part) wgradPart_.resizeAsync((uint32_t)part, s);
+    nn::launch_relu_bias(dY, Y, dPb_.devPtr(), nvox, L.cout, grad_.devPtr() + L.b, s);
+    nn::launch_conv3_wgrad(dPb_.devPtr(), X, grad_.devPtr() + L.w, wgradPart_.devPtr(), n, L.cin, L.cout, s);
     if (dX) nn::launch_conv3_dgrad(dPb_.devPtr(), params_.devPtr() + L.w, WT_.devPtr(), dX, n, L.cin, L.cout, s);
 }
 

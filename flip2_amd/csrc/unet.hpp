@@ -75,7 +75,7 @@ public:
 
 private:
     void conv(int layer, const uint16_t* X, uint16_t* Y, const nn::ConvMask& cm, hipStream_t s);
-    void convBackward(int layer, float* dY, const uint16_t* Y, const uint16_t* X, float* dX, hipStream_t s);
+    void convBackward(int layer, const float* dY, const uint16_t* Y, const uint16_t* X, float* dX, hipStream_t s);
 
     int n_, n1_, n2_;
     hipStream_t stream_;
@@ -100,6 +100,7 @@ private:
     // gradients (FP32)
     DeviceVec<float> gd0_, gc0_, gu0_, gd1_, gc1_, gu1_, gb2_, ga2_, gp1_, gb1_, ga1_, gp0_, gb0_, ga0_;
     DeviceVec<double> red_;
+    DeviceVec<float> wgradPart_;    // the weight gradient's sums per workgroup
     DeviceVec<uint16_t> dPb_, WT_;  // BF16 gradient of the current layer, transposed weights
     // set by applyActive for its forward: the first layer reads the solver's
     // slots, the head writes them

@@ -1060,34 +1060,37 @@ tile_lists_kernel(const uint8_t* __restrict__ cur, const uint8_t* __restrict__ p
     }
 }
 
-// g <- g * (act > 0) in place, and a BF16 copy of the result for the
-// MFMA gradient kernels.
-__global__ void relu_mask_bf16_kernel(float* __restrict__ g, const uint16_t* __restrict__ act,
-                                      uint16_t* __restrict__ gb, long long count) {
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= count) return;
-    float v = g[i];
-    if (!(bf2f(act[i]) > 0.f)) v = 0.f;
-    g[i] = v;
-    gb[i] = f2bf(v);
-}
-
-// dB[c] += sum_v g[v][c]: grid-stride partial sums per workgroup, one atomic
-// per channel per workgroup.
-__global__ void __launch_bounds__(256) bias_grad_kernel(const float* __restrict__ g, long long nvox, int C,
+// gb = BF16 of g * (act > 0), the gradient before the activation, and
+// dB[c] += its FP32 sum over the voxels: grid-stride partial sums per
+// workgroup, one atomic per channel per workgroup.  Memory-bound: g and act
+// are read once and gb written once (masking in place and summing in a second
+// pass over the FP32 gradient took 7.0 + 10.3 us per layer at 64^3).
+__global__ void __launch_bounds__(256) relu_bias_kernel(const float* __restrict__ g, const uint16_t* __restrict__ act,
+                                                        uint16_t* __restrict__ gb, long long nvox, int C,
                                                         float* __restrict__ dB) {
-    __shared__ float s_acc[256];
-    const int c = threadIdx.x % C;
-    const int lanesPerC = 256 / C;  // C divides 256 (16, 32 or 64)
-    const int sub = threadIdx.x / C;
-    float acc = 0.f;
-    for (long long v = (long long)blockIdx.x * lanesPerC + sub; v < nvox; v += (long long)gridDim.x * lanesPerC)
-        acc += g[v * C + c];
-    s_acc[threadIdx.x] = acc;
+    __shared__ float s_acc[256][4];
+    const int quads = C / 4;  // C divides 256 (16, 32 or 64): a thread's channels are fixed
+    const int q = threadIdx.x % quads, sub = threadIdx.x / quads, rows = 256 / quads;
+    float acc[4] = {0.f, 0.f, 0.f, 0.f};
+    for (long long v = (long long)blockIdx.x * rows + sub; v < nvox; v += (long long)gridDim.x * rows) {
+        const float4 x = *reinterpret_cast<const float4*>(g + v * C + 4 * q);
+        const uint2 y = *reinterpret_cast<const uint2*>(act + v * C + 4 * q);
+        const float t[4] = {x.x, x.y, x.z, x.w};
+        const uint32_t yw[4] = {y.x << 16, y.x & 0xffff0000u, y.y << 16, y.y & 0xffff0000u};
+        float m[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            m[e] = __uint_as_float(yw[e]) > 0.f ? t[e] : 0.f;
+            acc[e] += m[e];
+        }
+        *reinterpret_cast<uint2*>(gb + v * C + 4 * q) = make_uint2(f2bf2(m[0], m[1]), f2bf2(m[2], m[3]));
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) s_acc[threadIdx.x][e] = acc[e];
     __syncthreads();
-    if (threadIdx.x < C) {
+    if ((int)threadIdx.x < C) {
         float t = 0.f;
-        for (int k = 0; k < lanesPerC; ++k) t += s_acc[k * C + threadIdx.x];
+        for (int k = 0; k < rows; ++k) t += s_acc[k * quads + threadIdx.x / 4][threadIdx.x & 3];
         atomicAdd(&dB[threadIdx.x], t);
     }
 }
@@ -1102,108 +1105,157 @@ __global__ void transpose_weights_kernel(const float* __restrict__ W, uint16_t* 
     WT[i] = f2bf(W[((26 - t) * cout + co) * cin + ci]);
 }
 
-// dW[tap][co][ci] += sum_v dP[v][co] X[v + off(tap)][ci] on MFMA: a GEMM with
-// M = COUT, N = CIN and the voxels as the reduction dimension.  Workgroup
-// (chunk, tap): 128-voxel slices of its chunk are staged in LDS transposed
-// ([channel][voxel], rows padded against bank conflicts) so each lane's four
-// consecutive voxels are one 8-byte read; each wave owns some of the 16x16
-// output tiles; the chunk's partial sums go to dW with FP32 atomics.
-template <int CIN, int COUT>
+// Weight gradient, dW[tap][co][ci] += sum_v dP[v][co] X[v + off(tap)][ci]:
+// GEMMs on v_mfma_f32_16x16x32_bf16 with M = 16 output channels, N = 16 input
+// channels and K = 32 voxels (two x-rows of a tile), FP32 accumulation.
+//
+// A workgroup owns one 16 x 16 channel pair and walks 16 x 4 x 4 tiles of
+// voxels.  A tile's gradient and its input with the one-voxel halo are staged
+// in LDS once, transposed to [channel][row][x], and serve all 27 taps (a
+// workgroup per tap re-read both from memory 27 times, two bytes per lane and
+// load, and added its sums with atomics: 2.3 ms for the ten layers at 64^3;
+// this form 0.20 ms, and 0.05 ms for the sums).  Wave w takes the tile's z-slice w and keeps the 27 taps'
+// accumulators (108 registers) over all its tiles.  A lane's B fragment is
+// eight x-consecutive inputs of one channel: five dwords from the aligned
+// start give the three x-taps, the middle one by shifting a halfword.  The
+// next tile is loaded into registers during the MFMAs.  Row and channel
+// strides (12 and 436 or 132 dwords) put the sixteen lanes of a fragment read
+// on different banks.  Each workgroup stores its sums (no atomics);
+// conv3_wgrad_sum_kernel adds them in workgroup order.
+constexpr int kWgXRow = 12, kWgXCh = 436, kWgPRow = 8, kWgPCh = 132;  // LDS strides in dwords
+constexpr int kWgOut = 27 * 256;                                      // sums of one channel pair
+constexpr int kWgXItems = 9 * 36 * 2;                                 // voxel pairs x halo rows x 8-channel halves
+
+// a & m, per dword
+__device__ inline uint4 keep4(uint4 a, bool keep) {
+    const uint32_t m = keep ? 0xffffffffu : 0u;
+    return make_uint4(a.x & m, a.y & m, a.z & m, a.w & m);
+}
+// Two voxels' eight channels (a: the lower x) as eight dwords of one channel
+// each, stored `stride` dwords apart.
+__device__ inline void store_pairs(uint32_t* dst, int stride, const uint4& a, const uint4& b) {
+    const uint32_t aw[4] = {a.x, a.y, a.z, a.w}, bw[4] = {b.x, b.y, b.z, b.w};
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        dst[(2 * j) * stride] = (aw[j] & 0xffffu) | (bw[j] << 16);
+        dst[(2 * j + 1) * stride] = (aw[j] >> 16) | (bw[j] & 0xffff0000u);
+    }
+}
+
 __global__ void __launch_bounds__(256)
-conv3_wgrad_mfma_kernel(const uint16_t* __restrict__ dP, const uint16_t* __restrict__ X, float* __restrict__ dW,
-                        int n, long long chunk) {
-    constexpr int KV = 128, KP = KV + 4;
-    constexpr int MT = COUT / 16, NT = CIN / 16, T = MT * NT;
-    // with fewer than 4 output tiles the waves also split the reduction
-    constexpr int KSPLIT = T >= 4 ? 1 : (T == 1 ? 4 : (T == 2 ? 2 : 1));
-    constexpr int TW = KSPLIT > 1 ? 1 : (T + 3) / 4;
-    __shared__ __align__(16) uint16_t sP[COUT * KP];
-    __shared__ __align__(16) uint16_t sX[CIN * KP];
-    const int tap = blockIdx.y;
-    const int dx = tap % 3 - 1, dy = (tap / 3) % 3 - 1, dz = tap / 9 - 1;
-    const long long nvox = (long long)n * n * n;
-    const long long vBeg = (long long)blockIdx.x * chunk;
-    const long long vEnd = vBeg + chunk < nvox ? vBeg + chunk : nvox;
+conv3_wgrad_tile_kernel(const uint16_t* __restrict__ dP, const uint16_t* __restrict__ X, float* __restrict__ part,
+                        int n, int cin, int cout, int tilesX, int tilesY, int tiles) {
+    union Lds {
+        struct {
+            uint32_t x[16 * kWgXCh], p[16 * kWgPCh];
+        } in;
+        float sum[4][9 * 256];
+    };
+    __shared__ __align__(16) Lds lds;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int col = lane & 15, kq = lane >> 4;
-    v4f acc[TW];
+    const int nt = cin / 16, mp = (int)blockIdx.y / nt, np = (int)blockIdx.y % nt;  // this workgroup's channel blocks
+    v4f acc[27];
 #pragma unroll
-    for (int t = 0; t < TW; ++t) acc[t] = v4f{0.f, 0.f, 0.f, 0.f};
-    for (long long vb = vBeg; vb < vEnd; vb += KV) {
-        __syncthreads();
-        for (int i = threadIdx.x; i < KV * COUT; i += 256) {
-            const int k = i / COUT, c = i % COUT;
-            const long long v = vb + k;
-            sP[c * KP + k] = v < vEnd ? dP[v * COUT + c] : (uint16_t)0;
+    for (int t = 0; t < 27; ++t) acc[t] = v4f{0.f, 0.f, 0.f, 0.f};
+    uint4 px[3][2], pp[2];
+    // (every load is in bounds, its coordinates clamped into the grid; a voxel
+    // outside is zeroed)
+    auto at = [&](const uint16_t* A, int C, int c0, int x, int y, int z) {
+        const bool in = x >= 0 && y >= 0 && z >= 0 && x < n && y < n && z < n;
+        const int xc = min(max(x, 0), n - 1), yc = min(max(y, 0), n - 1), zc = min(max(z, 0), n - 1);
+        return keep4(*reinterpret_cast<const uint4*>(A + (((size_t)zc * n + yc) * n + xc) * C + c0), in);
+    };
+    auto load = [&](int tile) {
+        const int bx = (tile % tilesX) * kTX, by = ((tile / tilesX) % tilesY) * kTY, bz = (tile / (tilesX * tilesY)) * kTZ;
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            const int t = min((int)threadIdx.x + 256 * k, kWgXItems - 1);
+            const int half = t & 1, q = t >> 1, x = bx - 1 + 2 * (q % 9), row = q / 9;
+            const int y = by - 1 + row % 6, z = bz - 1 + row / 6;
+#pragma unroll
+            for (int e = 0; e < 2; ++e) px[k][e] = at(X, cin, 16 * np + 8 * half, x + e, y, z);
         }
-        for (int i = threadIdx.x; i < KV * CIN; i += 256) {
-            const int k = i / CIN, c = i % CIN;
-            const long long v = vb + k;
-            uint16_t xv = 0;
-            if (v < vEnd) {
-                const int x = (int)(v % n) + dx, y = (int)((v / n) % n) + dy, z = (int)(v / ((long long)n * n)) + dz;
-                if (x >= 0 && y >= 0 && z >= 0 && x < n && y < n && z < n)
-                    xv = X[(((long long)z * n + y) * n + x) * CIN + c];
+        const int t = (int)threadIdx.x, half = t & 1, q = t >> 1, x = bx + 2 * (q & 7), row = q >> 3;
+#pragma unroll
+        for (int e = 0; e < 2; ++e) pp[e] = at(dP, cout, 16 * mp + 8 * half, x + e, by + (row & 3), bz + (row >> 2));
+    };
+    auto store = [&] {
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            const int t = (int)threadIdx.x + 256 * k;
+            if (t < kWgXItems) {
+                const int half = t & 1, q = t >> 1;
+                store_pairs(&lds.in.x[8 * half * kWgXCh + (q / 9) * kWgXRow + q % 9], kWgXCh, px[k][0], px[k][1]);
             }
-            sX[c * KP + k] = xv;
         }
+        const int t = (int)threadIdx.x, half = t & 1, q = t >> 1;
+        store_pairs(&lds.in.p[8 * half * kWgPCh + (q >> 3) * kWgPRow + (q & 7)], kWgPCh, pp[0], pp[1]);
+    };
+    int tile = (int)blockIdx.x;  // (the grid has at most `tiles` workgroups per pair)
+    load(tile);
+    for (; tile < tiles; tile += (int)gridDim.x) {
+        __syncthreads();  // every wave is done with the previous tile
+        store();
         __syncthreads();
-        if (KSPLIT > 1) {
-            const int t = wave % T, ks = wave / T;
-            const int m = t / NT, nn = t % NT;
-            if (ks < KSPLIT) {
+        if (tile + (int)gridDim.x < tiles) load(tile + (int)gridDim.x);
 #pragma unroll
-                for (int k0 = 16 * ks; k0 < KV; k0 += 16 * KSPLIT) {
-                    const v4s a = *reinterpret_cast<const v4s*>(&sP[(16 * m + col) * KP + k0 + 4 * kq]);
-                    const v4s b = *reinterpret_cast<const v4s*>(&sX[(16 * nn + col) * KP + k0 + 4 * kq]);
-                    acc[0] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc[0], 0, 0, 0);
+        for (int yp = 0; yp < 2; ++yp) {
+            const int y0 = 2 * yp + (kq >> 1);  // this lane's row of the pair
+            const v8bf a = __builtin_bit_cast(
+                v8bf, *reinterpret_cast<const uint4*>(&lds.in.p[col * kWgPCh + (4 * wave + y0) * kWgPRow + 4 * (kq & 1)]));
+#pragma unroll
+            for (int dz = 0; dz < 3; ++dz)
+#pragma unroll
+                for (int dy = 0; dy < 3; ++dy) {
+                    const uint32_t* src =
+                        &lds.in.x[col * kWgXCh + ((wave + dz) * 6 + y0 + dy) * kWgXRow + 4 * (kq & 1)];
+                    const uint4 d = *reinterpret_cast<const uint4*>(src);
+                    const uint32_t d4 = src[4];
+                    const uint4 mid = make_uint4(__builtin_amdgcn_alignbit(d.y, d.x, 16), __builtin_amdgcn_alignbit(d.z, d.y, 16),
+                                                 __builtin_amdgcn_alignbit(d.w, d.z, 16), __builtin_amdgcn_alignbit(d4, d.w, 16));
+                    const int t = 3 * dy + 9 * dz;
+                    acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, __builtin_bit_cast(v8bf, d), acc[t], 0, 0, 0);
+                    acc[t + 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, __builtin_bit_cast(v8bf, mid), acc[t + 1], 0, 0, 0);
+                    acc[t + 2] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                        a, __builtin_bit_cast(v8bf, make_uint4(d.y, d.z, d.w, d4)), acc[t + 2], 0, 0, 0);
                 }
-            }
-        } else {
-#pragma unroll
-            for (int k0 = 0; k0 < KV; k0 += 16) {
-#pragma unroll
-                for (int tt = 0; tt < TW; ++tt) {
-                    const int t = wave + 4 * tt;
-                    if (t >= T) break;
-                    const int m = t / NT, nn = t % NT;
-                    const v4s a = *reinterpret_cast<const v4s*>(&sP[(16 * m + col) * KP + k0 + 4 * kq]);
-                    const v4s b = *reinterpret_cast<const v4s*>(&sX[(16 * nn + col) * KP + k0 + 4 * kq]);
-                    acc[tt] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc[tt], 0, 0, 0);
-                }
-            }
         }
     }
-    if (KSPLIT > 1) {
-        // sum the KSPLIT partial tiles through LDS (reusing sP), then one
-        // wave per tile adds the result to dW
-        __syncthreads();
-        float* red = reinterpret_cast<float*>(sP);  // 4 waves x 256 floats <= sizeof(sP)
+    // the four waves' sums, nine taps at a time
+    float* out = part + ((size_t)blockIdx.y * gridDim.x + blockIdx.x) * kWgOut;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) red[wave * 256 + (4 * kq + r) * 16 + col] = acc[0][r];
+    for (int g = 0; g < 3; ++g) {
         __syncthreads();
-        if (wave < T) {
-            const int t = wave, m = t / NT, nn = t % NT;
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                float v = 0.f;
-                for (int ks = 0; ks < KSPLIT; ++ks) v += red[(t + ks * T) * 256 + (4 * kq + r) * 16 + col];
-                const int co = 16 * m + 4 * kq + r, ci = 16 * nn + col;
-                atomicAdd(&dW[((size_t)tap * COUT + co) * CIN + ci], v);
-            }
-        }
-        return;
+        for (int t = 0; t < 9; ++t)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) lds.sum[wave][t * 256 + (4 * kq + r) * 16 + col] = acc[9 * g + t][r];
+        __syncthreads();
+        for (int i = threadIdx.x; i < 9 * 256; i += 256)
+            out[9 * 256 * g + i] = (lds.sum[0][i] + lds.sum[1][i]) + (lds.sum[2][i] + lds.sum[3][i]);
     }
+}
+
+// dW += the workgroups' sums of each channel pair, in a fixed order (thread
+// row r adds the workgroups r, r + 16, ..., then the rows are added in turn).
+__global__ void __launch_bounds__(1024)
+conv3_wgrad_sum_kernel(const float* __restrict__ part, float* __restrict__ dW, int cin, int cout, int groups) {
+    __shared__ float s_row[16][64];
+    const int o = (int)threadIdx.x & 63, row = (int)threadIdx.x >> 6;
+    const int i = (int)blockIdx.x * 64 + o;  // 27 * 256 outputs: whole workgroups
+    const int nt = cin / 16, mp = (int)blockIdx.y / nt, np = (int)blockIdx.y % nt;
+    const float* src = part + (size_t)blockIdx.y * groups * kWgOut + i;
+    float s = 0.f;
+    for (int g = row; g < groups; g += 16) s += src[(size_t)g * kWgOut];
+    s_row[row][o] = s;
+    __syncthreads();
+    if (row == 0) {
+        float t = 0.f;
 #pragma unroll
-    for (int tt = 0; tt < TW; ++tt) {
-        const int t = wave + 4 * tt;
-        if (t >= T) break;
-        const int m = t / NT, nn = t % NT;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int co = 16 * m + 4 * kq + r, ci = 16 * nn + col;
-            atomicAdd(&dW[((size_t)tap * COUT + co) * CIN + ci], acc[tt][r]);
-        }
+        for (int r = 0; r < 16; ++r) t += s_row[r][o];
+        const int tap = i >> 8, co = 16 * mp + ((i >> 4) & 15), ci = 16 * np + (i & 15);
+        dW[((size_t)tap * cout + co) * cin + ci] += t;
     }
 }
 
@@ -1523,40 +1575,39 @@ void launch_conv3_dgrad(const uint16_t* dPb, const float* W32, uint16_t* WT, flo
     throw Error(kErrArgument, "conv3 dgrad: unsupported channel pair");
 }
 
-void launch_conv3_wgrad(const uint16_t* dPb, const float* dP, const uint16_t* X, float* dW, float* dB, int n, int cin,
-                        int cout, hipStream_t s) {
-    const long long nvox = (long long)n * n * n;
-    // bias: column sums of dP
-    const int bblocks = (int)std::min<long long>(1024, (nvox + 255) / 256);
-    FLIP2_KERNEL(bias_grad_kernel, dim3(bblocks), dim3(256), 0, s, dP, nvox, cout, dB);
-    FLIP2_LAUNCH_CHECK();
-    // chunks: enough workgroups to fill the GPU, few enough that the atomics
-    // (27 * cout * cin per chunk) stay around 4M
-    long long chunks = std::max<long long>(1, 4000000LL / (27LL * cin * cout));
-    chunks = std::min<long long>(chunks, (nvox + 127) / 128);
-    long long chunk = (nvox + chunks - 1) / chunks;
-    chunk = (chunk + 127) / 128 * 128;
-    chunks = (nvox + chunk - 1) / chunk;
-#define WGRAD_CASE(CI, CO)                                                                                      \
-    if (cin == CI && cout == CO) {                                                                              \
-        FLIP2_KERNEL((conv3_wgrad_mfma_kernel<CI, CO>), dim3((unsigned)chunks, 27), dim3(256), 0, s, dPb, X, \
-                           dW, n, chunk);                                                                       \
-        FLIP2_LAUNCH_CHECK();                                                                                   \
-        return;                                                                                                 \
-    }
-    WGRAD_CASE(16, 16)
-    WGRAD_CASE(16, 32)
-    WGRAD_CASE(32, 32)
-    WGRAD_CASE(32, 64)
-    WGRAD_CASE(64, 64)
-    WGRAD_CASE(96, 32)
-    WGRAD_CASE(48, 16)
-#undef WGRAD_CASE
-    throw Error(kErrArgument, "conv3 wgrad: unsupported channel pair");
+namespace {
+// Workgroups per channel pair: one per CU over all pairs, at most one per
+// tile (each stores 27 KB of sums, which the summing kernel reads back).
+int wgrad_groups(int n, int cin, int cout) {
+    const int pairs = (cin / 16) * (cout / 16);
+    return (int)std::min<long long>(conv_tiles(n), std::max(1, (256 + pairs - 1) / pairs));
+}
+}  // namespace
+
+size_t conv3_wgrad_part_floats(int n, int cin, int cout) {
+    return (size_t)(cin / 16) * (cout / 16) * wgrad_groups(n, cin, cout) * kWgOut;
 }
 
-void launch_relu_mask_bf16(float* g, const uint16_t* act, uint16_t* gb, long long count, hipStream_t s) {
-    FLIP2_KERNEL(relu_mask_bf16_kernel, g1(count, 256), dim3(256), 0, s, g, act, gb, count);
+void launch_conv3_wgrad(const uint16_t* dPb, const uint16_t* X, float* dW, float* part, int n, int cin, int cout,
+                        hipStream_t s) {
+    FLIP2_REQUIRE(cin % 16 == 0 && cout % 16 == 0 && cin > 0 && cout > 0, kErrArgument,
+                  "conv3 wgrad: unsupported channel pair");
+    uint32_t tilesX = 0, tilesY = 0;
+    conv_tile_dims(n, tilesX, tilesY);
+    const int groups = wgrad_groups(n, cin, cout);
+    const unsigned pairs = (unsigned)((cin / 16) * (cout / 16));
+    FLIP2_KERNEL(conv3_wgrad_tile_kernel, dim3((unsigned)groups, pairs), dim3(256), 0, s, dPb, X, part, n, cin, cout,
+                 (int)tilesX, (int)tilesY, (int)conv_tiles(n));
+    FLIP2_LAUNCH_CHECK();
+    FLIP2_KERNEL(conv3_wgrad_sum_kernel, dim3(kWgOut / 64, pairs), dim3(1024), 0, s, part, dW, cin, cout, groups);
+    FLIP2_LAUNCH_CHECK();
+}
+
+void launch_relu_bias(const float* g, const uint16_t* act, uint16_t* gb, long long nvox, int C, float* dB,
+                      hipStream_t s) {
+    FLIP2_REQUIRE(C % 4 == 0 && C > 0 && 256 % C == 0, kErrArgument, "activation gradient: unsupported channel count");
+    const int blocks = (int)std::min<long long>(512, (nvox * C + 4095) / 4096);
+    FLIP2_KERNEL(relu_bias_kernel, dim3(blocks), dim3(256), 0, s, g, act, gb, nvox, C, dB);
     FLIP2_LAUNCH_CHECK();
 }
 void launch_avgpool(const uint16_t* X, uint16_t* P, int n, int C, hipStream_t s) {

@@ -95,11 +95,14 @@ uint32_t conv_tiles(int n);
 // BF16 scratch) receives the transposed, mirrored weights.
 void launch_conv3_dgrad(const uint16_t* dPb, const float* W32, uint16_t* WT, float* dX, int n, int cin, int cout,
                         hipStream_t s);
-// dW += sum_v dP (x) X(v + tap) (MFMA on dPb and X), dB += sum_v dP (FP32).
-void launch_conv3_wgrad(const uint16_t* dPb, const float* dP, const uint16_t* X, float* dW, float* dB, int n, int cin,
-                        int cout, hipStream_t s);
-// g <- g * (act > 0) in place; gb = BF16 copy.
-void launch_relu_mask_bf16(float* g, const uint16_t* act, uint16_t* gb, long long count, hipStream_t s);
+// dW += sum_v dP (x) X(v + tap) (MFMA on dPb and X); part:
+// conv3_wgrad_part_floats floats of scratch.
+size_t conv3_wgrad_part_floats(int n, int cin, int cout);
+void launch_conv3_wgrad(const uint16_t* dPb, const uint16_t* X, float* dW, float* part, int n, int cin, int cout,
+                        hipStream_t s);
+// gb = BF16 of g * (act > 0); dB += its FP32 sums over the voxels.
+void launch_relu_bias(const float* g, const uint16_t* act, uint16_t* gb, long long nvox, int C, float* dB,
+                      hipStream_t s);
 void launch_avgpool(const uint16_t* X, uint16_t* P, int n, int C, hipStream_t s);
 void launch_avgpool_bwd(const float* dP, float* dX, int n, int C, hipStream_t s);  // dX += ...
 void launch_upcat(const uint16_t* A, const uint16_t* B, uint16_t* U, int n, int Ca, int Cb, hipStream_t s);
