@@ -665,13 +665,9 @@ void UNet::backward(const float* dOut, hipStream_t s) {
                         grad_.devPtr() + headW_, grad_.devPtr() + headB_, N0, 16, s);
     convBackward(9, gd0_.devPtr(), d0_.devPtr(), c0_.devPtr(), gc0_.devPtr(), s);
     convBackward(8, gc0_.devPtr(), c0_.devPtr(), u0_.devPtr(), gu0_.devPtr(), s);
-    nn::launch_zero_f32(gd1_.devPtr(), N1 * 32, s);
-    nn::launch_zero_f32(gb0_.devPtr(), N0 * 16, s);
     nn::launch_upcat_bwd(gu0_.devPtr(), gd1_.devPtr(), gb0_.devPtr(), n_, 32, 16, s);
     convBackward(7, gd1_.devPtr(), d1_.devPtr(), c1_.devPtr(), gc1_.devPtr(), s);
     convBackward(6, gc1_.devPtr(), c1_.devPtr(), u1_.devPtr(), gu1_.devPtr(), s);
-    nn::launch_zero_f32(gb2_.devPtr(), N2 * 64, s);
-    nn::launch_zero_f32(gb1_.devPtr(), N1 * 32, s);
     nn::launch_upcat_bwd(gu1_.devPtr(), gb2_.devPtr(), gb1_.devPtr(), n1_, 64, 32, s);
     convBackward(5, gb2_.devPtr(), b2_.devPtr(), a2_.devPtr(), ga2_.devPtr(), s);
     convBackward(4, ga2_.devPtr(), a2_.devPtr(), p1_.devPtr(), gp1_.devPtr(), s);

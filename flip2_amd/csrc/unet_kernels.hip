@@ -1281,57 +1281,68 @@ __global__ void avgpool_kernel(const uint16_t* __restrict__ X, uint16_t* __restr
 }
 
 __global__ void avgpool_bwd_kernel(const float* __restrict__ dP, float* __restrict__ dX, int n, int C) {
+    const int c4 = C / 4;  // four channels per thread
     const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    const long long total = (long long)n * n * n * C;
+    const long long total = (long long)n * n * n * c4;
     if (i >= total) return;
-    const int c = (int)(i % C);
-    const long long v = i / C;
+    const int c = (int)(i % c4) * 4;
+    const long long v = i / c4;
     const int x = (int)(v % n), y = (int)((v / n) % n), z = (int)(v / ((long long)n * n));
     const int nc = n / 2;
-    dX[i] += 0.125f * dP[(((long long)(z / 2) * nc + y / 2) * nc + x / 2) * C + c];
+    const float4 g = *reinterpret_cast<const float4*>(dP + (((long long)(z / 2) * nc + y / 2) * nc + x / 2) * C + c);
+    float4* d = reinterpret_cast<float4*>(dX) + i;
+    const float4 o = *d;
+    *d = make_float4(fmaf(0.125f, g.x, o.x), fmaf(0.125f, g.y, o.y), fmaf(0.125f, g.z, o.z), fmaf(0.125f, g.w, o.w));
 }
 
 // U[v][0:Ca] = A[parent(v)] (nearest upsampling), U[v][Ca:Ca+Cb] = B[v].
+// Eight channels (16 bytes) per thread; Ca and Cb are multiples of 8.
 __global__ void upcat_kernel(const uint16_t* __restrict__ A, const uint16_t* __restrict__ Bsk, uint16_t* __restrict__ U,
                              int n, int Ca, int Cb) {
-    const int C = Ca + Cb;
+    const int C8 = (Ca + Cb) / 8;
     const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    const long long total = (long long)n * n * n * C;
-    if (i >= total) return;
-    const int c = (int)(i % C);
-    const long long v = i / C;
+    if (i >= (long long)n * n * n * C8) return;
+    const int c = (int)(i % C8) * 8;
+    const long long v = i / C8;
+    const uint16_t* src;
     if (c < Ca) {
         const int x = (int)(v % n), y = (int)((v / n) % n), z = (int)(v / ((long long)n * n));
         const int nc = n / 2;
-        U[i] = A[(((long long)(z / 2) * nc + y / 2) * nc + x / 2) * Ca + c];
+        src = A + (((long long)(z / 2) * nc + y / 2) * nc + x / 2) * Ca + c;
     } else {
-        U[i] = Bsk[v * Cb + (c - Ca)];
+        src = Bsk + v * Cb + (c - Ca);
     }
+    reinterpret_cast<uint4*>(U)[i] = *reinterpret_cast<const uint4*>(src);
 }
 
-// dA[parent][c] += sum of the 8 children's dU[child][c]; dB[v][c] += dU[v][Ca+c]
+// Gradients of the concatenation: dA = the sum of dU over the children, dBsk
+// = dU's skip channels.  Four channels (16 bytes) per thread.
 __global__ void upcat_bwd_kernel(const float* __restrict__ dU, float* __restrict__ dA, float* __restrict__ dBsk, int n,
                                  int Ca, int Cb) {
-    const int C = Ca + Cb;
+    const int C = Ca + Cb, a4 = Ca / 4, b4 = Cb / 4;
     const int nc = n / 2;
     const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    const long long coarse = (long long)nc * nc * nc * Ca;
-    const long long fine = (long long)n * n * n * Cb;
+    const long long coarse = (long long)nc * nc * nc * a4;
+    const long long fine = (long long)n * n * n * b4;
     if (i < coarse) {
-        const int c = (int)(i % Ca);
-        const long long vp = i / Ca;
+        const int c = (int)(i % a4) * 4;
+        const long long vp = i / a4;
         const int x = (int)(vp % nc), y = (int)((vp / nc) % nc), z = (int)(vp / ((long long)nc * nc));
-        float s = 0.f;
+        float4 t[8];
+#pragma unroll
         for (int k = 0; k < 8; ++k) {
             const int xf = 2 * x + (k & 1), yf = 2 * y + ((k >> 1) & 1), zf = 2 * z + (k >> 2);
-            s += dU[(((long long)zf * n + yf) * n + xf) * C + c];
+            t[k] = *reinterpret_cast<const float4*>(dU + (((long long)zf * n + yf) * n + xf) * C + c);
         }
-        dA[i] += s;
+        float4 s = t[0];
+#pragma unroll
+        for (int k = 1; k < 8; ++k) s = make_float4(s.x + t[k].x, s.y + t[k].y, s.z + t[k].z, s.w + t[k].w);
+        reinterpret_cast<float4*>(dA)[i] = s;
     } else if (i < coarse + fine) {
         const long long j = i - coarse;
-        const int c = (int)(j % Cb);
-        const long long v = j / Cb;
-        dBsk[j] += dU[v * C + Ca + c];
+        const int c = (int)(j % b4) * 4;
+        const long long v = j / b4;
+        reinterpret_cast<float4*>(dBsk)[j] = *reinterpret_cast<const float4*>(dU + v * C + Ca + c);
     }
 }
 
@@ -1351,29 +1362,36 @@ __global__ void head_fwd_kernel(const uint16_t* __restrict__ X, const float* __r
 __global__ void __launch_bounds__(256)
 head_bwd_kernel(const float* __restrict__ dOut, const uint16_t* __restrict__ X, const float* __restrict__ w,
                 const uint8_t* __restrict__ mask, const float* __restrict__ scale, float* __restrict__ dX,
-                float* __restrict__ dw, float* __restrict__ db, long long nvox, int C) {
-    __shared__ float s_red[17][256];
-    const long long v = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    float g = 0.f;
-    float part[16];
-    for (int c = 0; c < 16; ++c) part[c] = 0.f;
-    if (v < nvox) {
-        g = mask[v] ? dOut[v] * scale[0] : 0.f;
-        for (int c = 0; c < C; ++c) {
-            dX[v * C + c] = g * w[c];
-            part[c] = g * bf2f(X[v * C + c]);
-        }
+                float* __restrict__ dw, float* __restrict__ db, long long nvox) {
+    // four threads per voxel, four channels each; grid-stride, so a workgroup
+    // adds its sums once (1024 workgroups' atomics on 17 words were most of
+    // the 46 us at 64^3)
+    __shared__ float s_red[4][4][5];
+    const int q = threadIdx.x & 3, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const float4 wq = *reinterpret_cast<const float4*>(w + 4 * q);
+    float part[5] = {0.f, 0.f, 0.f, 0.f, 0.f};  // the four channels', and (q == 0) the bias's
+    for (long long v = (long long)blockIdx.x * 64 + (threadIdx.x >> 2); v < nvox; v += (long long)gridDim.x * 64) {
+        const float g = mask[v] ? dOut[v] * scale[0] : 0.f;
+        const uint2 x = *reinterpret_cast<const uint2*>(X + v * 16 + 4 * q);
+        *reinterpret_cast<float4*>(dX + v * 16 + 4 * q) = make_float4(g * wq.x, g * wq.y, g * wq.z, g * wq.w);
+        part[0] = fmaf(g, __uint_as_float(x.x << 16), part[0]);
+        part[1] = fmaf(g, __uint_as_float(x.x & 0xffff0000u), part[1]);
+        part[2] = fmaf(g, __uint_as_float(x.y << 16), part[2]);
+        part[3] = fmaf(g, __uint_as_float(x.y & 0xffff0000u), part[3]);
+        part[4] += g;
     }
-    for (int c = 0; c < 16; ++c) s_red[c][threadIdx.x] = part[c];
-    s_red[16][threadIdx.x] = g;
+#pragma unroll
+    for (int e = 0; e < 5; ++e)
+        for (int d = 32; d >= 4; d >>= 1) part[e] += __shfl_xor(part[e], d, 64);
+    if (lane < 4)
+#pragma unroll
+        for (int e = 0; e < 5; ++e) s_red[wave][lane][e] = part[e];
     __syncthreads();
-    for (int s = 128; s >= 1; s >>= 1) {
-        if ((int)threadIdx.x < s)
-            for (int c = 0; c < 17; ++c) s_red[c][threadIdx.x] += s_red[c][threadIdx.x + s];
-        __syncthreads();
+    if (threadIdx.x < 17) {
+        const int qq = threadIdx.x < 16 ? (int)threadIdx.x >> 2 : 0, e = threadIdx.x < 16 ? (int)threadIdx.x & 3 : 4;
+        const float t = (s_red[0][qq][e] + s_red[1][qq][e]) + (s_red[2][qq][e] + s_red[3][qq][e]);
+        atomicAdd(threadIdx.x < 16 ? &dw[threadIdx.x] : db, t);
     }
-    if (threadIdx.x < (unsigned)C) atomicAdd(&dw[threadIdx.x], s_red[threadIdx.x][0]);
-    if (threadIdx.x == 16) atomicAdd(db, s_red[16][0]);
 }
 
 // Adam on FP32 master weights, BF16 copy refreshed.
@@ -1556,13 +1574,21 @@ void launch_conv3_dgrad(const uint16_t* dPb, const float* W32, uint16_t* WT, flo
     FLIP2_LAUNCH_CHECK();
     (void)nvox;
     const dim3 grid = conv_grid(n);
-    // the forward kernel with the roles of the channel counts swapped
-#define DGRAD_CASE(CI, CO)                                                                                      \
-    if (cin == CI && cout == CO) {                                                                              \
-        FLIP2_KERNEL((conv3_fwd_kernel<CO, CI, 1>), grid, dim3(256), 0, s, dPb, (const uint16_t*)nullptr, WT,  \
-                           (const float*)nullptr, (uint16_t*)nullptr, dX, n, 0, HeadArgs{}, ConvMask{});       \
-        FLIP2_LAUNCH_CHECK();                                                                                   \
-        return;                                                                                                 \
+    // the forward kernel with the roles of the channel counts swapped; on
+    // small grids a workgroup per 16 output channels (64 -> 64 channels at
+    // 16^3: 16 workgroups in 52 us, 64 in 17; a large grid fills the chip
+    // with workgroups that stage their input once for all channels)
+    const bool split = grid.x * grid.y * grid.z < 2048u;
+#define DGRAD_LAUNCH(CI, CO, SP)                                                                              \
+    FLIP2_KERNEL((conv3_fwd_kernel<CO, CI, 1, 0, SP>), dim3(grid.x * SP, grid.y, grid.z), dim3(256), 0, s, dPb, \
+                 (const uint16_t*)nullptr, WT, (const float*)nullptr, (uint16_t*)nullptr, dX, n, 0, HeadArgs{}, \
+                 ConvMask{})
+#define DGRAD_CASE(CI, CO)                         \
+    if (cin == CI && cout == CO) {                 \
+        if (split) DGRAD_LAUNCH(CI, CO, CI / 16);  \
+        else DGRAD_LAUNCH(CI, CO, 1);              \
+        FLIP2_LAUNCH_CHECK();                      \
+        return;                                    \
     }
     DGRAD_CASE(16, 16)
     DGRAD_CASE(16, 32)
@@ -1572,6 +1598,7 @@ void launch_conv3_dgrad(const uint16_t* dPb, const float* W32, uint16_t* WT, flo
     DGRAD_CASE(96, 32)
     DGRAD_CASE(48, 16)
 #undef DGRAD_CASE
+#undef DGRAD_LAUNCH
     throw Error(kErrArgument, "conv3 dgrad: unsupported channel pair");
 }
 
@@ -1616,17 +1643,20 @@ void launch_avgpool(const uint16_t* X, uint16_t* P, int n, int C, hipStream_t s)
     FLIP2_LAUNCH_CHECK();
 }
 void launch_avgpool_bwd(const float* dP, float* dX, int n, int C, hipStream_t s) {
-    const long long total = (long long)n * n * n * C;
+    FLIP2_REQUIRE(C % 4 == 0, kErrArgument, "pooling gradient: channels in fours");
+    const long long total = (long long)n * n * n * (C / 4);
     FLIP2_KERNEL(avgpool_bwd_kernel, g1(total, 256), dim3(256), 0, s, dP, dX, n, C);
     FLIP2_LAUNCH_CHECK();
 }
 void launch_upcat(const uint16_t* A, const uint16_t* B, uint16_t* U, int n, int Ca, int Cb, hipStream_t s) {
-    const long long total = (long long)n * n * n * (Ca + Cb);
+    FLIP2_REQUIRE(Ca % 8 == 0 && Cb % 8 == 0, kErrArgument, "concatenation: channels in eights");
+    const long long total = (long long)n * n * n * ((Ca + Cb) / 8);
     FLIP2_KERNEL(upcat_kernel, g1(total, 256), dim3(256), 0, s, A, B, U, n, Ca, Cb);
     FLIP2_LAUNCH_CHECK();
 }
 void launch_upcat_bwd(const float* dU, float* dA, float* dB, int n, int Ca, int Cb, hipStream_t s) {
-    const long long total = (long long)(n / 2) * (n / 2) * (n / 2) * Ca + (long long)n * n * n * Cb;
+    FLIP2_REQUIRE(Ca % 4 == 0 && Cb % 4 == 0, kErrArgument, "concatenation gradient: channels in fours");
+    const long long total = (long long)(n / 2) * (n / 2) * (n / 2) * (Ca / 4) + (long long)n * n * n * (Cb / 4);
     FLIP2_KERNEL(upcat_bwd_kernel, g1(total, 256), dim3(256), 0, s, dU, dA, dB, n, Ca, Cb);
     FLIP2_LAUNCH_CHECK();
 }
@@ -1637,8 +1667,9 @@ void launch_head_fwd(const uint16_t* X, const float* w, const float* b, const ui
 }
 void launch_head_bwd(const float* dOut, const uint16_t* X, const float* w, const uint8_t* mask, const float* scale,
                      float* dX, float* dw, float* db, long long nvox, int C, hipStream_t s) {
-    FLIP2_REQUIRE(C <= 16, kErrArgument, "head: at most 16 channels");
-    FLIP2_KERNEL(head_bwd_kernel, g1(nvox, 256), dim3(256), 0, s, dOut, X, w, mask, scale, dX, dw, db, nvox, C);
+    FLIP2_REQUIRE(C == 16, kErrArgument, "head: 16 channels");
+    const int blocks = (int)std::min<long long>(256, (nvox + 63) / 64);
+    FLIP2_KERNEL(head_bwd_kernel, dim3(blocks), dim3(256), 0, s, dOut, X, w, mask, scale, dX, dw, db, nvox);
     FLIP2_LAUNCH_CHECK();
 }
 void launch_adam(float* w, const float* g, float* m, float* v, uint16_t* wbf, int count, float lr, float b1, float b2,

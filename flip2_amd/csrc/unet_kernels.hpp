@@ -106,7 +106,7 @@ void launch_relu_bias(const float* g, const uint16_t* act, uint16_t* gb, long lo
 void launch_avgpool(const uint16_t* X, uint16_t* P, int n, int C, hipStream_t s);
 void launch_avgpool_bwd(const float* dP, float* dX, int n, int C, hipStream_t s);  // dX += ...
 void launch_upcat(const uint16_t* A, const uint16_t* B, uint16_t* U, int n, int Ca, int Cb, hipStream_t s);
-void launch_upcat_bwd(const float* dU, float* dA, float* dB, int n, int Ca, int Cb, hipStream_t s);  // +=
+void launch_upcat_bwd(const float* dU, float* dA, float* dB, int n, int Ca, int Cb, hipStream_t s);  // writes dA and dB
 void launch_head_fwd(const uint16_t* X, const float* w, const float* b, const uint8_t* mask, const float* scale,
                      float* out, long long nvox, int C, hipStream_t s);
 void launch_head_bwd(const float* dOut, const uint16_t* X, const float* w, const uint8_t* mask, const float* scale,
