@@ -6,12 +6,14 @@
 // Per sort:
 //   1. one histogram kernel counts the 8-bit digits of every pass at once
 //      and clears the look-back words;
-//   2. a small kernel turns the counts into per-pass digit offsets;
-//   3. one kernel per pass: each tile (256 lanes x 16..32 keys) ranks its keys by digit with
+//   2. one kernel per pass: each tile (256 lanes x 4..32 keys) ranks its keys by digit with
 //      64-lane ballot matching (stable within the wave), publishes its digit
-//      counts, resolves its global digit bases by per-digit decoupled
-//      look-back over earlier tiles, stages the keys in LDS in sorted order
-//      and writes them out in digit runs.
+//      counts, resolves its global digit bases by the exclusive scan of the
+//      pass's counts and per-digit decoupled look-back over earlier tiles,
+//      stages the keys in LDS in sorted order and writes them out in digit
+//      runs.
+// Up to 8192 keys are sorted by one workgroup in one launch, all passes in
+// its LDS (sort_small_kernel).
 // A stable LSD sort has a unique output, so keys and the permutation match
 // the reference's bit for bit.
 #include "sort.hpp"
@@ -24,12 +26,8 @@ namespace {
 
 constexpr int kSortThreads = 256;             // 4 waves
 constexpr int kSortWaves = kSortThreads / 64;
-constexpr int kMinSortItems = 16;             // keys per lane of the smallest tile
-constexpr int kMinSortTile = kSortThreads * kMinSortItems;  // 4096
 constexpr int kRadix = 256;
 constexpr int kHistThreads = 256;
-constexpr int kHistItems = 32;                // keys per thread per chunk in the histogram kernel
-constexpr uint32_t kHistChunk = kHistThreads * kHistItems;  // 8192 keys
 constexpr int kLookback = 16;                 // earlier tiles whose status a digit loads per step
 constexpr uint32_t kDigitFlagShift = 30;
 constexpr uint32_t kDigitValueMask = (1u << kDigitFlagShift) - 1u;
@@ -37,21 +35,33 @@ constexpr uint32_t kDigitAggregate = 1u << kDigitFlagShift;
 constexpr uint32_t kDigitInclusive = 2u << kDigitFlagShift;
 constexpr int kMaxPasses = 4;
 
+// Keys per lane of a digit-pass tile.  Large sorts: fewer tiles and
+// look-backs, longer digit runs (32 measured fastest at millions of keys).
+// Small ones are a chain of latencies, and a tile's ranking is a chain over
+// its keys per lane: more, shorter tiles, as long as a look-back reaches the
+// first in a few steps (24 bits: 65536 keys 33 us with 4 keys per lane, 40
+// with 8, 49 with 16; 262144 keys 52, 53 and 57; 524288 keys 80, 63 and 64).
+constexpr int kManyKeys = 1 << 20, kFewKeys = 1 << 18;
+int sort_items(uint32_t n) { return n >= (uint32_t)kManyKeys ? 32 : n >= (uint32_t)kFewKeys ? 16 : 4; }
+
+constexpr int kSmallThreads = 1024;
+// Most keys of the one-workgroup sort: with 16 keys per lane it takes 52 us at
+// 16384 keys over 32 bits, the digit kernels 34.
+constexpr uint32_t kSmallKeys = 8 * kSmallThreads;
+
 struct SortLayout {
     uint32_t passes;
-    uint32_t tiles;       // tiles of the smallest tile size (sizes the status area)
-    size_t histOff, offsetOff, counterOff, statusOff, total;
+    size_t histOff, counterOff, statusOff, total;
 };
 
-SortLayout sort_layout(uint32_t n, uint32_t beginBit, uint32_t endBit) {
+SortLayout sort_layout(uint32_t n, uint32_t beginBit, uint32_t endBit, int items) {
     SortLayout L{};
     L.passes = (endBit > beginBit) ? ceil_div(endBit - beginBit, 8) : 0;
-    L.tiles = ceil_div(n ? n : 1, kMinSortTile);  // enough for every tile size
+    const uint32_t tiles = ceil_div(n ? n : 1, (uint32_t)items * kSortThreads);
     size_t off = 0;
-    L.histOff = off; off += (size_t)kMaxPasses * kRadix * sizeof(uint32_t);
-    L.offsetOff = off; off += (size_t)kMaxPasses * kRadix * sizeof(uint32_t);
+    L.histOff = off; off += (size_t)2 * kMaxPasses * kRadix * sizeof(uint32_t);
     L.counterOff = off; off += 256;
-    L.statusOff = off; off += (size_t)L.passes * L.tiles * kRadix * sizeof(uint32_t);
+    L.statusOff = off; off += (size_t)L.passes * tiles * kRadix * sizeof(uint32_t);
     L.total = off + 256;
     return L;
 }
@@ -66,10 +76,11 @@ __global__ void sort_clear_kernel(uint32_t* words, uint32_t count) {
     if (i < count) words[i] = 0;
 }
 
-// Digit histograms of every pass.  A workgroup counts one chunk of 8192 keys
-// in LDS (all of a thread's loads issued before its counting) and adds its
+// Digit histograms of every pass.  A workgroup counts one chunk of 256 ITEMS
+// keys in LDS (all of a thread's loads issued before its counting) and adds its
 // counts to the global histogram, one atomic per non-empty bin.  The same
 // launch clears the look-back status words of the passes.
+template <int ITEMS>
 __global__ void __launch_bounds__(kHistThreads)
 sort_histogram_kernel(const uint32_t* __restrict__ keys, uint32_t n, uint32_t beginBit, uint32_t endBit,
                       uint32_t passes, uint32_t* __restrict__ hist, uint32_t* __restrict__ clearWords,
@@ -78,11 +89,12 @@ sort_histogram_kernel(const uint32_t* __restrict__ keys, uint32_t n, uint32_t be
     for (int i = threadIdx.x; i < kMaxPasses * kRadix; i += kHistThreads) s_hist[i] = 0;
     for (uint32_t i = blockIdx.x * kHistThreads + threadIdx.x; i < clearCount; i += gridDim.x * kHistThreads)
         clearWords[i] = 0;
-    const uint32_t base = blockIdx.x * kHistChunk;
-    const bool vec = (reinterpret_cast<uintptr_t>(keys) & 15u) == 0 && base + kHistChunk <= n;
-    uint32_t key[kHistItems];
+    constexpr uint32_t kChunk = kHistThreads * ITEMS;
+    const uint32_t base = blockIdx.x * kChunk;
+    const bool vec = (reinterpret_cast<uintptr_t>(keys) & 15u) == 0 && base + kChunk <= n;
+    uint32_t key[ITEMS];
 #pragma unroll
-    for (int k = 0; k < kHistItems / 4; ++k) {
+    for (int k = 0; k < ITEMS / 4; ++k) {
         const uint32_t i = base + ((uint32_t)k * kHistThreads + threadIdx.x) * 4u;
         if (vec) {
             const uint4 v = *reinterpret_cast<const uint4*>(keys + i);
@@ -94,7 +106,7 @@ sort_histogram_kernel(const uint32_t* __restrict__ keys, uint32_t n, uint32_t be
     }
     __syncthreads();
 #pragma unroll
-    for (int k = 0; k < kHistItems / 4; ++k) {
+    for (int k = 0; k < ITEMS / 4; ++k) {
         const uint32_t i = base + ((uint32_t)k * kHistThreads + threadIdx.x) * 4u;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
@@ -125,23 +137,6 @@ sort_histogram_kernel(const uint32_t* __restrict__ keys, uint32_t n, uint32_t be
     }
 }
 
-// Exclusive scan of each pass's 256 digit counts (one workgroup, one wave
-// per pass).
-__global__ void sort_offsets_kernel(const uint32_t* __restrict__ hist, uint32_t passes,
-                                    uint32_t* __restrict__ offsets) {
-    const int lane = threadIdx.x & 63;
-    const uint32_t p = threadIdx.x >> 6;
-    if (p >= passes) return;
-    uint32_t carry = 0;
-    for (int chunk = 0; chunk < kRadix / 64; ++chunk) {
-        const uint32_t d = (uint32_t)chunk * 64u + (uint32_t)lane;
-        const uint32_t c = hist[p * kRadix + d];
-        const uint32_t incl = wave_inclusive_scan(c);
-        offsets[p * kRadix + d] = carry + incl - c;
-        carry += __shfl(incl, 63, 64);
-    }
-}
-
 __device__ inline uint32_t digit_status_load(const uint32_t* p) {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
@@ -153,14 +148,14 @@ template <int ITEMS>
 __global__ void __launch_bounds__(kSortThreads)
 sort_pass_kernel(const uint32_t* __restrict__ keysIn, const uint32_t* __restrict__ valsIn,
                  uint32_t* __restrict__ keysOut, uint32_t* __restrict__ valsOut, uint32_t n,
-                 uint32_t shift, uint32_t mask, const uint32_t* __restrict__ digitOffsets,
+                 uint32_t shift, uint32_t mask, const uint32_t* __restrict__ digitCounts,
                  uint32_t* __restrict__ status, uint32_t* __restrict__ counter) {
     __shared__ uint32_t s_keys[(ITEMS * kSortThreads)];
     __shared__ uint32_t s_vals[(ITEMS * kSortThreads)];
     __shared__ uint32_t s_wave[kSortWaves][kRadix];  // counts, then exclusive offsets across waves
     __shared__ uint32_t s_tileExcl[kRadix];
     __shared__ uint32_t s_globalBase[kRadix];
-    __shared__ uint32_t s_scanTmp[kSortWaves];
+    __shared__ uint32_t s_scanTmp[2][kSortWaves];
     __shared__ uint32_t s_tile;
 
     const int tid = threadIdx.x;
@@ -215,14 +210,24 @@ sort_pass_kernel(const uint32_t* __restrict__ keysIn, const uint32_t* __restrict
     uint32_t* myStatus = status + (size_t)tile * kRadix + d;
     digit_status_store(myStatus, (tile == 0 ? kDigitInclusive : kDigitAggregate) | tileCount);
 
-    // Exclusive scan of the tile counts over the 256 digits.
+    // Exclusive scans over the 256 digits of the tile's counts and of the
+    // whole pass's (the digits' offsets in the output).
+    uint32_t digitOffset = 0;
     {
         const uint32_t incl = wave_inclusive_scan(tileCount);
-        if (lane == 63) s_scanTmp[wave] = incl;
+        const uint32_t all = digitCounts[d], allIncl = wave_inclusive_scan(all);
+        if (lane == 63) {
+            s_scanTmp[0][wave] = incl;
+            s_scanTmp[1][wave] = allIncl;
+        }
         __syncthreads();
         uint32_t waveOff = 0;
-        for (int w = 0; w < wave; ++w) waveOff += s_scanTmp[w];
+        for (int w = 0; w < wave; ++w) {
+            waveOff += s_scanTmp[0][w];
+            digitOffset += s_scanTmp[1][w];
+        }
         s_tileExcl[d] = waveOff + incl - tileCount;
+        digitOffset += allIncl - all;
     }
 
     // Per-digit look-back over the earlier tiles, kLookback tiles per step:
@@ -255,7 +260,7 @@ sort_pass_kernel(const uint32_t* __restrict__ keysIn, const uint32_t* __restrict
         digit_status_store(myStatus, kDigitInclusive | (prefix + tileCount));
     }
     __syncthreads();
-    s_globalBase[d] = digitOffsets[d] + prefix - s_tileExcl[d];
+    s_globalBase[d] = digitOffset + prefix - s_tileExcl[d];
 
     // Stage in LDS in tile-sorted order.
 #pragma unroll
@@ -281,6 +286,101 @@ sort_pass_kernel(const uint32_t* __restrict__ keysIn, const uint32_t* __restrict
     }
 }
 
+// Every pass of a sort of at most 1024 ITEMS keys by one workgroup: keys and
+// values in registers, ranked as in sort_pass_kernel, scattered through LDS.
+// A chain of latencies: 4099 keys over 32 bits take 26 us in one launch, the
+// digit kernels' seven launches took 52.
+template <int ITEMS>
+__global__ void __launch_bounds__(kSmallThreads)
+sort_small_kernel(const uint32_t* __restrict__ keysIn, const uint32_t* __restrict__ valsIn,
+                  uint32_t* __restrict__ keysOut, uint32_t* __restrict__ valsOut, uint32_t n, uint32_t beginBit,
+                  uint32_t endBit) {
+    constexpr int kWaves = kSmallThreads / 64;
+    __shared__ uint32_t s_kv[2][ITEMS * kSmallThreads];
+    __shared__ uint32_t s_wave[kWaves][kRadix];
+    __shared__ uint32_t s_scanTmp[4];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const uint32_t waveBase = (uint32_t)wave * (64u * ITEMS) + (uint32_t)lane;
+    uint32_t key[ITEMS], val[ITEMS];
+#pragma unroll
+    for (int k = 0; k < ITEMS; ++k) {
+        const uint32_t i = waveBase + 64u * (uint32_t)k;
+        key[k] = i < n ? keysIn[i] : 0xffffffffu;
+        val[k] = i < n ? (valsIn ? valsIn[i] : i) : 0u;
+    }
+    const uint64_t ltMask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+    for (uint32_t shift = beginBit; shift < endBit; shift += 8u) {
+        const uint32_t mask = (1u << min(8u, endBit - shift)) - 1u;
+        for (int i = tid; i < kWaves * kRadix; i += kSmallThreads) (&s_wave[0][0])[i] = 0;
+        __syncthreads();
+        uint32_t rank[ITEMS];
+#pragma unroll
+        for (int k = 0; k < ITEMS; ++k) {
+            const bool valid = waveBase + 64u * (uint32_t)k < n;
+            const uint32_t d = digit_of(key[k], shift, mask);
+            uint64_t m = __ballot(valid);
+#pragma unroll
+            for (int b = 0; b < 8; ++b) {
+                const uint64_t bm = __ballot((d >> b) & 1u);
+                m &= ((d >> b) & 1u) ? bm : ~bm;
+            }
+            const uint64_t lower = m & ltMask;
+            const uint32_t before = s_wave[wave][d];
+            __builtin_amdgcn_wave_barrier();
+            if (valid && lower == 0) s_wave[wave][d] = before + (uint32_t)__popcll(m);
+            __builtin_amdgcn_wave_barrier();
+            rank[k] = before + (uint32_t)__popcll(lower);
+        }
+        __syncthreads();
+        // thread d < 256: the waves' exclusive offsets of digit d, after all
+        // smaller digits
+        uint32_t count = 0, incl = 0;
+        if (tid < kRadix) {
+#pragma unroll
+            for (int w = 0; w < kWaves; ++w) {
+                const uint32_t c = s_wave[w][tid];
+                s_wave[w][tid] = count;
+                count += c;
+            }
+            incl = wave_inclusive_scan(count);
+            if (lane == 63) s_scanTmp[wave] = incl;
+        }
+        __syncthreads();
+        if (tid < kRadix) {
+            uint32_t off = incl - count;
+            for (int w = 0; w < wave; ++w) off += s_scanTmp[w];
+#pragma unroll
+            for (int w = 0; w < kWaves; ++w) s_wave[w][tid] += off;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < ITEMS; ++k) {
+            if (waveBase + 64u * (uint32_t)k < n) {
+                const uint32_t pos = s_wave[wave][digit_of(key[k], shift, mask)] + rank[k];
+                s_kv[0][pos] = key[k];
+                s_kv[1][pos] = val[k];
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < ITEMS; ++k) {
+            const uint32_t i = waveBase + 64u * (uint32_t)k;
+            if (i < n) {
+                key[k] = s_kv[0][i];
+                val[k] = s_kv[1][i];
+            }
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < ITEMS; ++k) {
+        const uint32_t i = waveBase + 64u * (uint32_t)k;
+        if (i < n) {
+            keysOut[i] = key[k];
+            valsOut[i] = val[k];
+        }
+    }
+}
+
 }  // namespace
 
 uint32_t sort_passes(uint32_t beginBit, uint32_t endBit) {
@@ -289,23 +389,27 @@ uint32_t sort_passes(uint32_t beginBit, uint32_t endBit) {
 
 size_t sort_workspace_bytes(uint32_t n, uint32_t beginBit, uint32_t endBit) {
     if (endBit > 32) endBit = 32;
-    return sort_layout(n, beginBit, endBit).total;
+    // status words of 4096-key tiles, the shortest but for few keys, and enough
+    // for every smaller sort (a workspace outlives one length)
+    return std::max(sort_layout(n, beginBit, endBit, 16).total,
+                    sort_layout(std::min<uint32_t>(n, kFewKeys - 1), beginBit, endBit, 4).total);
 }
 
 void sort_pairs_u32(const uint32_t* keysIn, const uint32_t* valsIn, uint32_t* keysOut, uint32_t* valsOut,
                     uint32_t* keysAlt, uint32_t* valsAlt, uint32_t n, uint32_t beginBit, uint32_t endBit,
                     void* ws, size_t wsBytes, hipStream_t stream, hipEvent_t* passEvents, int itemsPerThread) {
-    // 32 keys per lane measured fastest at millions of keys (fewer tiles and
-    // look-backs, longer digit runs per tile); small inputs keep more tiles
-    const int items = itemsPerThread ? itemsPerThread : (n >= (1u << 20) ? 32 : 16);
-    FLIP2_REQUIRE(items == 16 || items == 24 || items == 32, kErrArgument, "sort: 16, 24 or 32 keys per lane");
+    int items = itemsPerThread ? itemsPerThread : sort_items(n);
+    // (a workspace that holds only the status words of 4096-key tiles will do)
+    if (!itemsPerThread && items == 4 && wsBytes < sort_layout(n, beginBit, endBit, 4).total) items = 16;
+    FLIP2_REQUIRE(items == 4 || items == 16 || items == 24 || items == 32, kErrArgument,
+                  "sort: 4, 16, 24 or 32 keys per lane");
     FLIP2_REQUIRE(endBit <= 32 && beginBit <= endBit, kErrArgument, "sort: bad bit range");
     FLIP2_REQUIRE(n < (1u << kDigitFlagShift), kErrRange, "sort: n must be below 2^30");
     FLIP2_REQUIRE(keysIn && keysOut && valsOut, kErrArgument, "sort: null buffer");
     FLIP2_REQUIRE(keysIn != keysOut && keysIn != keysAlt && (!valsIn || (valsIn != valsOut && valsIn != valsAlt)),
                   kErrArgument, "sort: inputs must not alias outputs");
     if (n == 0) return;
-    const SortLayout L = sort_layout(n, beginBit, endBit);
+    const SortLayout L = sort_layout(n, beginBit, endBit, items);
     FLIP2_REQUIRE(ws && wsBytes >= L.total, kErrArgument, "sort: workspace too small");
     if (L.passes == 0) {
         FLIP2_HIP(hipMemcpyAsync(keysOut, keysIn, (size_t)n * 4, hipMemcpyDeviceToDevice, stream));
@@ -319,9 +423,21 @@ void sort_pairs_u32(const uint32_t* keysIn, const uint32_t* valsIn, uint32_t* ke
         return;
     }
     FLIP2_REQUIRE(L.passes == 1 || (keysAlt && valsAlt), kErrArgument, "sort: alternate buffers required");
+    if (n <= kSmallKeys && !itemsPerThread) {
+        if (passEvents) FLIP2_HIP(hipEventRecord(passEvents[0], stream));
+        if (n <= 4u * kSmallThreads)
+            FLIP2_KERNEL(sort_small_kernel<4>, dim3(1), dim3(kSmallThreads), 0, stream, keysIn, valsIn, keysOut,
+                         valsOut, n, beginBit, endBit);
+        else
+            FLIP2_KERNEL(sort_small_kernel<8>, dim3(1), dim3(kSmallThreads), 0, stream, keysIn, valsIn, keysOut,
+                         valsOut, n, beginBit, endBit);
+        FLIP2_LAUNCH_CHECK();
+        if (passEvents)
+            for (uint32_t p = 0; p < L.passes; ++p) FLIP2_HIP(hipEventRecord(passEvents[p + 1], stream));
+        return;
+    }
     char* w = reinterpret_cast<char*>(ws);
     uint32_t* hist = reinterpret_cast<uint32_t*>(w + L.histOff);
-    uint32_t* offsets = reinterpret_cast<uint32_t*>(w + L.offsetOff);
     uint32_t* counters = reinterpret_cast<uint32_t*>(w + L.counterOff);
     uint32_t* status = reinterpret_cast<uint32_t*>(w + L.statusOff);
 
@@ -333,10 +449,13 @@ void sort_pairs_u32(const uint32_t* keysIn, const uint32_t* valsIn, uint32_t* ke
     FLIP2_KERNEL(sort_clear_kernel, dim3(ceil_div(headWords, 256)), dim3(256), 0, stream,
                        reinterpret_cast<uint32_t*>(w), headWords);
     FLIP2_LAUNCH_CHECK();
-    FLIP2_KERNEL(sort_histogram_kernel, dim3(ceil_div(n, kHistChunk)), dim3(kHistThreads), 0, stream, keysIn, n,
-                       beginBit, endBit, L.passes, hist, status, (uint32_t)(L.passes * passStride));
-    FLIP2_LAUNCH_CHECK();
-    FLIP2_KERNEL(sort_offsets_kernel, dim3(1), dim3(64 * kMaxPasses), 0, stream, hist, L.passes, offsets);
+    // chunks of 8192 keys, of 1024 for small sorts (whose time is a chunk's)
+    if (items > 4)
+        FLIP2_KERNEL(sort_histogram_kernel<32>, dim3(ceil_div(n, 32u * kHistThreads)), dim3(kHistThreads), 0, stream,
+                     keysIn, n, beginBit, endBit, L.passes, hist, status, (uint32_t)(L.passes * passStride));
+    else
+        FLIP2_KERNEL(sort_histogram_kernel<4>, dim3(ceil_div(n, 4u * kHistThreads)), dim3(kHistThreads), 0, stream,
+                     keysIn, n, beginBit, endBit, L.passes, hist, status, (uint32_t)(L.passes * passStride));
     FLIP2_LAUNCH_CHECK();
     if (passEvents) FLIP2_HIP(hipEventRecord(passEvents[0], stream));
 
@@ -353,13 +472,16 @@ void sort_pairs_u32(const uint32_t* keysIn, const uint32_t* valsIn, uint32_t* ke
         uint32_t* st = status + (size_t)p * passStride;
         if (items == 32)
             FLIP2_KERNEL(sort_pass_kernel<32>, dim3(ceil_div(n, 32u * kSortThreads)), dim3(kSortThreads), 0,
-                               stream, srcK, srcV, dstK, dstV, n, shift, mask, offsets + p * kRadix, st, counters + p);
+                               stream, srcK, srcV, dstK, dstV, n, shift, mask, hist + p * kRadix, st, counters + p);
         else if (items == 24)
             FLIP2_KERNEL(sort_pass_kernel<24>, dim3(ceil_div(n, 24u * kSortThreads)), dim3(kSortThreads), 0,
-                               stream, srcK, srcV, dstK, dstV, n, shift, mask, offsets + p * kRadix, st, counters + p);
+                               stream, srcK, srcV, dstK, dstV, n, shift, mask, hist + p * kRadix, st, counters + p);
+        else if (items == 4)
+            FLIP2_KERNEL(sort_pass_kernel<4>, dim3(ceil_div(n, 4u * kSortThreads)), dim3(kSortThreads), 0,
+                               stream, srcK, srcV, dstK, dstV, n, shift, mask, hist + p * kRadix, st, counters + p);
         else
             FLIP2_KERNEL(sort_pass_kernel<16>, dim3(ceil_div(n, 16u * kSortThreads)), dim3(kSortThreads), 0,
-                               stream, srcK, srcV, dstK, dstV, n, shift, mask, offsets + p * kRadix, st, counters + p);
+                               stream, srcK, srcV, dstK, dstV, n, shift, mask, hist + p * kRadix, st, counters + p);
         FLIP2_LAUNCH_CHECK();
         if (passEvents) FLIP2_HIP(hipEventRecord(passEvents[p + 1], stream));
         srcK = dstK;
