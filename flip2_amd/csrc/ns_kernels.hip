@@ -277,20 +277,34 @@ struct P2GShared {
     uint32_t wave[4];
 };
 
+// t 2^32 rounded to a 64-bit integer, for 0 <= t < 2^32 (five instructions;
+// the general float to integer conversion takes seven, eleven for a signed
+// result).  The fraction is exact and below 1 - 2^-25, so lo does not carry.
+__device__ inline unsigned long long fixed64(float t) {
+    const uint32_t hi = (uint32_t)t;
+    const uint32_t lo = (uint32_t)rintf(__builtin_amdgcn_fractf(t) * 4294967296.0f);
+    return ((unsigned long long)hi << 32) | lo;
+}
+
 // Scatter of brick bb (index `brick`) into sh.w, sh.m (cleared here) by the
 // 256 threads of the workgroup; scaleW, scaleM: the fixed-point scales.
-// Ends with the sums complete and visible to the workgroup.
+// Ends with the sums complete and visible to the workgroup.  C >= 0: of that
+// face component only.  The kernel is bound by its instruction issue (~24
+// corners per particle, with the conversions to fixed point; every particle
+// is visited by its own brick's workgroup and, near a side, its neighbours'),
+// then by the LDS atomics.
 // occ (may be null): brick occupancy flags; a run in a brick without
 // particles is empty without reading cellStart (which then need only hold
 // the cells of occupied bricks).
+template <int C = -1>
 __device__ inline void p2g_scatter_brick(P2GShared& sh, const int bb[3], uint32_t brick, const float4* __restrict__ rec,
                                          const uint32_t* __restrict__ cellStart, Grid g, uint32_t nbX, uint32_t nbY,
                                          uint32_t nbZ, const uint32_t* __restrict__ stats, float& scaleW,
                                          float& scaleM, const uint8_t* __restrict__ occ = nullptr) {
     const uint32_t tid = threadIdx.x;
-    for (uint32_t t = tid; t < 1536u; t += 256u) {
-        (&sh.w[0][0])[t] = 0ull;
-        (&sh.m[0][0])[t] = 0ull;
+    for (uint32_t t = tid; t < (C < 0 ? 1536u : 512u); t += 256u) {
+        (&sh.w[C < 0 ? 0 : C][0])[t] = 0ull;
+        (&sh.m[C < 0 ? 0 : C][0])[t] = 0ull;
     }
     // run table and its exclusive scan
     uint32_t first = 0, cnt = 0;
@@ -329,6 +343,7 @@ __device__ inline void p2g_scatter_brick(P2GShared& sh, const int bb[3], uint32_
     const int em = vmax > 0.f ? ilogbf(bound * vmax) + 1 : ew;
     scaleM = ldexpf(1.0f, min(62 - em, 126));
 
+    const float unitW = scaleW * 0x1p-32f, unitM = scaleM * 0x1p-32f;
     const double inv = 1.0 / (double)g.cellSize;
     const double org[3] = {(double)g.negX + (double)(bb[0] * 8) * (double)g.cellSize,
                            (double)g.negY + (double)(bb[1] * 8) * (double)g.cellSize,
@@ -377,7 +392,7 @@ __device__ inline void p2g_scatter_brick(P2GShared& sh, const int bb[3], uint32_
                                 (float)(((double)r0.z - org[2]) * inv)};
             const float vel[3] = {r0.w, r1.x, r1.y};
 #pragma unroll
-            for (int c = 0; c < 3; ++c) {
+            for (int c = C < 0 ? 0 : C; c < (C < 0 ? 3 : C + 1); ++c) {
                 int bs[3];
                 float t1[3];
 #pragma unroll
@@ -387,7 +402,9 @@ __device__ inline void p2g_scatter_brick(P2GShared& sh, const int bb[3], uint32_
                     bs[d] = (int)f;
                     t1[d] = v - f;
                 }
-                const float mv = vel[c] * scaleM;
+                const float mv = fabsf(vel[c]) * unitM;
+                const uint32_t sg = (uint32_t)(__float_as_int(vel[c]) >> 31);  // the momentum's sign
+                const unsigned long long sign = ((unsigned long long)sg << 32) | sg;
 #pragma unroll
                 for (int ax = 0; ax < 2; ++ax) {
                     const int li = bs[0] + ax;
@@ -404,8 +421,8 @@ __device__ inline void p2g_scatter_brick(P2GShared& sh, const int bb[3], uint32_
                             if ((unsigned)lk >= 8u) continue;
                             const float wt = wab * (bz ? t1[2] : 1.f - t1[2]);
                             const int node = lk * 64 + lj * 8 + li;
-                            atomicAdd(&sh.w[c][node], (unsigned long long)__float2ull_rn(wt * scaleW));
-                            atomicAdd(&sh.m[c][node], (unsigned long long)__float2ll_rn(wt * mv));
+                            atomicAdd(&sh.w[c][node], fixed64(wt * unitW));
+                            atomicAdd(&sh.m[c][node], (fixed64(wt * mv) ^ sign) - sign);
                         }
                     }
                 }
@@ -434,6 +451,7 @@ p2g_brick_kernel(const float4* __restrict__ rec, const uint32_t* __restrict__ ce
     __shared__ P2GShared sh;
     const uint32_t tid = threadIdx.x;
     const uint32_t perXcd = (numBricks + 7u) >> 3;
+    // gridDim.y == 3: a workgroup per brick and face component
     const uint32_t order = (blockIdx.x & 7u) * perXcd + (blockIdx.x >> 3);
     if (order >= numBricks) return;
     const uint32_t nbX = g.sizeX >> 3, nbY = g.sizeY >> 3, nbZ = g.sizeZ >> 3;
@@ -449,13 +467,21 @@ p2g_brick_kernel(const float4* __restrict__ rec, const uint32_t* __restrict__ ce
     }
     const uint32_t brick = ((uint32_t)bb[2] * nbY + (uint32_t)bb[1]) * nbX + (uint32_t)bb[0];
     float scaleW, scaleM;
-    p2g_scatter_brick(sh, bb, brick, rec, cellStart, g, nbX, nbY, nbZ, stats, scaleW, scaleM);
+    int c0 = 0, c1 = 3;
+    if (gridDim.y == 3u) {
+        c0 = (int)blockIdx.y;
+        c1 = c0 + 1;
+        if (c0 == 0) p2g_scatter_brick<0>(sh, bb, brick, rec, cellStart, g, nbX, nbY, nbZ, stats, scaleW, scaleM);
+        else if (c0 == 1) p2g_scatter_brick<1>(sh, bb, brick, rec, cellStart, g, nbX, nbY, nbZ, stats, scaleW, scaleM);
+        else p2g_scatter_brick<2>(sh, bb, brick, rec, cellStart, g, nbX, nbY, nbZ, stats, scaleW, scaleM);
+    } else {
+        p2g_scatter_brick(sh, bb, brick, rec, cellStart, g, nbX, nbY, nbZ, stats, scaleW, scaleM);
+    }
     float* out[3] = {U, V, W};
     float* outW[3] = {WU, WV, WW};
     const double iw = 1.0 / (double)scaleW, im = 1.0 / (double)scaleM;
     for (uint32_t t = tid; t < 512u; t += 256u) {
-#pragma unroll
-        for (int c = 0; c < 3; ++c) {
+        for (int c = c0; c < c1; ++c) {
             double ws;
             out[c][brick * 512u + t] = p2g_face(sh, c, t, iw, im, ws);
             if (outW[c]) outW[c][brick * 512u + t] = (float)ws;
@@ -631,7 +657,10 @@ empty_faces_kernel(const uint8_t* __restrict__ touched, const uint8_t* __restric
 // XCD each octant, i.e. most of a blob's particles to one or two XCDs).  A
 // workgroup takes the next entry of its XCD's share from that XCD's counter
 // (counters[xcd], zero at launch), one entry ahead, so workgroups with
-// light bricks take more of them.
+// light bricks take more of them.  With at most a third as many entries as
+// workgroups, a workgroup takes one face component of one entry (the same
+// sums): a full brick's particles through one workgroup are what a small
+// scene's transfer waits for (48 bricks, 13800 particles: 178 -> 36 us).
 __global__ void __launch_bounds__(256)
 p2g_prepare_kernel(const uint32_t* __restrict__ list, const uint32_t* __restrict__ count,
                    const float4* __restrict__ rec, const uint32_t* __restrict__ cellStart, Grid g,
@@ -646,6 +675,40 @@ p2g_prepare_kernel(const uint32_t* __restrict__ list, const uint32_t* __restrict
     const uint32_t xcd = blockIdx.x & 7u;  // workgroups are dealt to the XCDs round robin
     float* F[3] = {U, V, W};
     float* F0[3] = {U0, V0, W0};
+    // the prepared faces of components [c0, c1) of the scattered brick
+    auto write_faces = [&](uint32_t brick, const int bb[3], float scaleW, float scaleM, int c0, int c1) {
+        const double iw = 1.0 / (double)scaleW, im = 1.0 / (double)scaleM;
+        for (uint32_t t = threadIdx.x; t < 512u; t += 256u) {
+            float in[3] = {0.f, 0.f, 0.f};
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                double ws;
+                if (c >= c0 && c < c1) in[c] = p2g_face(sh, c, t, iw, im, ws);
+            }
+            const int gc[3] = {bb[0] * 8 + (int)(t & 7u), bb[1] * 8 + (int)((t >> 3) & 7u), bb[2] * 8 + (int)(t >> 6)};
+            float saved[3], out[3];
+            prepare_cell_faces(in, gc, g, solid, box, gdt, nbX, nbY, saved, out);
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                if (c < c0 || c >= c1) continue;
+                F0[c][brick * 512u + t] = saved[c];
+                F[c][brick * 512u + t] = out[c];
+            }
+        }
+    };
+    if (3u * total <= gridDim.x) {
+        const uint32_t e = blockIdx.x / 3u;
+        if (e >= total) return;
+        const int c = (int)(blockIdx.x % 3u);
+        const uint32_t brick = list[e];
+        const int bb[3] = {(int)(brick % nbX), (int)((brick / nbX) % nbY), (int)(brick / (nbX * nbY))};
+        float scaleW, scaleM;
+        if (c == 0) p2g_scatter_brick<0>(sh, bb, brick, rec, cellStart, g, nbX, nbY, nbZ, stats, scaleW, scaleM, occ);
+        else if (c == 1) p2g_scatter_brick<1>(sh, bb, brick, rec, cellStart, g, nbX, nbY, nbZ, stats, scaleW, scaleM, occ);
+        else p2g_scatter_brick<2>(sh, bb, brick, rec, cellStart, g, nbX, nbY, nbZ, stats, scaleW, scaleM, occ);
+        write_faces(brick, bb, scaleW, scaleM, c, c + 1);
+        return;
+    }
     if (threadIdx.x == 0) s_next = atomicAdd(&counters[xcd], 1u);
     __syncthreads();
     for (uint32_t m = s_next;; m = s_next) {
@@ -658,23 +721,7 @@ p2g_prepare_kernel(const uint32_t* __restrict__ list, const uint32_t* __restrict
         const int bb[3] = {(int)(brick % nbX), (int)((brick / nbX) % nbY), (int)(brick / (nbX * nbY))};
         float scaleW, scaleM;
         p2g_scatter_brick(sh, bb, brick, rec, cellStart, g, nbX, nbY, nbZ, stats, scaleW, scaleM, occ);
-        const double iw = 1.0 / (double)scaleW, im = 1.0 / (double)scaleM;
-        for (uint32_t t = threadIdx.x; t < 512u; t += 256u) {
-            float in[3];
-#pragma unroll
-            for (int c = 0; c < 3; ++c) {
-                double ws;
-                in[c] = p2g_face(sh, c, t, iw, im, ws);
-            }
-            const int gc[3] = {bb[0] * 8 + (int)(t & 7u), bb[1] * 8 + (int)((t >> 3) & 7u), bb[2] * 8 + (int)(t >> 6)};
-            float saved[3], out[3];
-            prepare_cell_faces(in, gc, g, solid, box, gdt, nbX, nbY, saved, out);
-#pragma unroll
-            for (int c = 0; c < 3; ++c) {
-                F0[c][brick * 512u + t] = saved[c];
-                F[c][brick * 512u + t] = out[c];
-            }
-        }
+        write_faces(brick, bb, scaleW, scaleM, 0, 3);
         __syncthreads();  // the next brick clears the sums; s_next is written
     }
 }
@@ -754,7 +801,12 @@ void launch_p2g(const float4* sortedRec, const uint32_t* cellStart, Grid g, cons
     const bool pow2 = (nbX & (nbX - 1)) == 0;
     const int morton = (nbX == nbY && nbY == nbZ && pow2 && nbX <= 1024) ? 1 : 0;
     const uint32_t blocks = ((numBricks + 7u) >> 3) * 8u;
-    FLIP2_KERNEL(p2g_brick_kernel, dim3(blocks), dim3(256), 0, s, sortedRec, cellStart, g, numBricks, morton,
+    // few bricks, as long as all workgroups are resident together: one per
+    // component too, so that a heavy brick's particles do not go through one
+    // workgroup alone; with more bricks the runs would be read three times
+    // for workgroups that only wait
+    const unsigned parts = 3u * blocks <= resident_groups(p2g_brick_kernel, 256) ? 3u : 1u;
+    FLIP2_KERNEL(p2g_brick_kernel, dim3(blocks, parts), dim3(256), 0, s, sortedRec, cellStart, g, numBricks, morton,
                        stats, U, V, W, WU, WV, WW);
     FLIP2_LAUNCH_CHECK();
 }
@@ -785,8 +837,10 @@ void launch_p2g_prepare(const float4* sortedRec, const uint32_t* sortedKeys, uin
     FLIP2_KERNEL(empty_faces_kernel, dim3((numBricks + 63u) / 64u), dim3(256), 0, s, t.touched, prep.full ? nullptr : t.prevTouched,
                  numBricks, g, prep.solid, prep.box, prep.gdt, U, V, W, prep.U0, prep.V0, prep.W0);
     FLIP2_LAUNCH_CHECK();
-    // as many workgroups as the CUs hold at once (registers and LDS), 8 per XCD row
-    const uint32_t groups = std::min<uint32_t>(resident_groups(p2g_prepare_kernel, 256), 8u * ((numBricks + 7u) >> 3));
+    // as many workgroups as the CUs hold at once (registers and LDS), 8 per XCD
+    // row; at most one per brick and component
+    const uint32_t groups =
+        std::min<uint32_t>(resident_groups(p2g_prepare_kernel, 256), 8u * ((3u * numBricks + 7u) >> 3));
     FLIP2_KERNEL(zero_u32_kernel, dim3(1), dim3(64), 0, s, t.counters, 8u);
     FLIP2_LAUNCH_CHECK();
     FLIP2_KERNEL(p2g_prepare_kernel, dim3(groups), dim3(256), 0, s, t.list, t.count, sortedRec, cellStart, g, stats,
