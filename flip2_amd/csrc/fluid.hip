@@ -46,7 +46,6 @@ constexpr uint32_t kMaxCheckEvery = 1u << 16;
 // ~30 us per iteration), and the 64-bit words its workgroups publish (six
 // for each of at most 256).
 constexpr uint32_t kResidentCap = 16384;
-constexpr uint32_t kResidentWords = 6 * 256;
 
 // One validator for every way a configuration enters the simulation
 // (creation, set_config, snapshot load).
@@ -527,7 +526,7 @@ FluidSim::ResidentEnd FluidSim::residentRefinement(uint32_t na, const ns::Reside
     FLIP2_HIP(hipGetDevice(&dev));
     const uint64_t last = (uint64_t)residentNumber_ + 2u * (uint64_t)limit + 4u;
     if (residentNumber_ == 0 || last > 0xffffffffull) {
-        ns::launch_fill_f64(words_.devPtr(), kResidentWords, 0.0, stream_);
+        ns::launch_fill_f64(words_.devPtr(), (uint32_t)ns::resident_words(), 0.0, stream_);
         ns::launch_fill_f64(scal_.devPtr() + 8, 2, 0.0, stream_);
         residentNumber_ = 1;
     }
@@ -602,12 +601,12 @@ SolveStats FluidSim::solveOnce(int prec, uint32_t capIn) {
     const bool perIteration = capture_ || (timer && timer->asksFor("cg_"));
     const ns::ResidentShape shape = !flex && !perIteration && residentOk_ && cap <= kResidentCap
                                         ? ns::resident_shape(na, !jac)
-                                        : ns::ResidentShape{0, 0};
+                                        : ns::ResidentShape{};
     const bool resident = shape.groups > 0;
     if (resident) {
         const size_t want = ns::resident_face_floats(na);
         if (faces_.size() < want) faces_.resizeAsync((uint32_t)ns::resident_face_floats(slotCapacity_), stream_);
-        if (words_.size() < kResidentWords) words_.resizeAsync(kResidentWords, stream_), residentNumber_ = 0;
+        if (words_.size() < (uint32_t)ns::resident_words()) words_.resizeAsync((uint32_t)ns::resident_words(), stream_), residentNumber_ = 0;
     } else {
         FLIP2_HIP(hipMemcpyAsync(r64_.devPtr(), b64_.devPtr(), (size_t)cells * sizeof(double),
                                  hipMemcpyDeviceToDevice, stream_));

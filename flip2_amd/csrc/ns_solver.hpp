@@ -123,22 +123,25 @@ struct CgResident {
     const double* r64;
     double* x64;
     float* faces;     // resident_face_floats(na)
-    uint64_t* words;  // 6 per workgroup, zero before the first launch
+    uint64_t* words;  // resident_words(), zero before the first launch
     uint32_t* result;
     uint32_t na;
     uint32_t groups;
     uint32_t limit;
     uint32_t polls;   // reads of a wait between workgroups before it is given up
     uint32_t number;  // of the first sum: larger by 2 limit + 2 than the previous launch's on these words
+    uint32_t pause;   // before a wait's first read, in 64 clocks (set at launch)
     double thr2;
 };
 // Workgroups and waves per workgroup for na slots; no groups where they do
 // not fit the chip at once.
 struct ResidentShape {
     uint32_t groups, waves;
+    bool wide;  // one slot per wave (else four)
 };
 ResidentShape resident_shape(uint32_t na, bool mic);
 size_t resident_face_floats(uint32_t na);
+size_t resident_words();
 // Held from a resident launch until its end: two of them at once could each
 // hold CUs that the other waits for.
 std::mutex& resident_mutex(int device);

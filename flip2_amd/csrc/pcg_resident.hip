@@ -6,14 +6,17 @@
 // for large systems, two summing kernels).  The vectors of up to ~11000 slots
 // fit the chip's registers and LDS, so here an iteration moves only the
 // slots' faces (1.5 KB out and in per slot) and two grid-wide sums.  Per
-// iteration, two-kernel form -> this one: 160 slots Jacobi 14.5 -> 6.9 us,
-// 1370 slots 19.6 -> 8.9 (Jacobi), 25.6 -> 12.1 (MIC(0)), 4122 slots
-// 33.6 -> 12.5 and 45.4 -> 16.4, 9194 slots 54.7 -> 20.5 and 68.9 -> 26.7.
-// What bounds it: below ~1000 slots the chain of one wave's instructions and
-// the latency of the two sums; above, the waves' instruction issue (~2400
-// per iteration for four slots with MIC(0), half of them the sweeps).
+// iteration of a solve, two-kernel form -> this one: 160 slots Jacobi 14.5 ->
+// 4.3 us, MIC(0) 18.9 -> 6.7; 960 slots 18.5 -> 5.5 and 22.6 -> 7.6; 2383
+// slots 21.9 -> 6.9 and 31.7 -> 9.8; 4122 slots 33.6 -> 10.1 and 45.4 -> 13.7;
+// 9196 slots 54.5 -> 21.4 and 68.6 -> 22.9.
+// What bounds it: up to ~2000 slots the latency of the two sums (a write
+// and a read through memory each, ~1.5 us) and, with MIC(0), the chain of the
+// sweeps' 44 steps; above, the waves' instruction issue (~2400 per iteration
+// for four slots with MIC(0), half of them the sweeps).
 //
-// Layout.  A wave holds four slots, one per row of 16 lanes.  Lane 8 J + i of
+// Layout of large systems (pcg_resident_kernel; pcg_wide_kernel, one slot per
+// wave, has its own below).  A wave holds four slots, one per row of 16 lanes.  Lane 8 J + i of
 // a row holds the cells (i, j = 4 J + b, k), b = 0..3, k = 0..7, of its slot:
 // 32 cells per vector.  Register [b][m] holds k = (m - i - j) mod 8, so cells
 // with the same i + j + k (mod 8) -- one anti-diagonal plane of the MIC(0)
@@ -34,12 +37,15 @@
 // carry 32 bits of a double and the sum's number, with relaxed agent-scope
 // stores (written through to memory: L2 is per XCD), and reads all the
 // others' until their numbers match; it adds them in workgroup order, so all
-// get the same double.  The faces are written through and waited for before
-// the words that announce them.  A workgroup waits for all others, so the
-// launch needs every workgroup on the chip at once: the grid is one workgroup
-// per CU at most, launches of one process take turns (resident_mutex), and
-// every wait is bounded -- if it runs out (another process holds CUs), the
-// kernel ends, reports it, and the caller solves with the two-kernel form.
+// get the same double.  The words are published in eight copies, one for the
+// workgroups of each XCD: 256 workgroups reading the same lines wait for each
+// other (960 slots, Jacobi: 6.2 -> 5.7 us per iteration).  The faces are
+// written through and waited for before the words that announce them.  A
+// workgroup waits for all others, so the launch needs every workgroup on the
+// chip at once: the grid is one workgroup per CU at most, launches of one
+// process take turns (resident_mutex), and every wait is bounded -- if it
+// runs out (another process holds CUs), the kernel ends, reports it, and the
+// caller solves with the two-kernel form.
 #include "ns_solver.hpp"
 
 #include <cstddef>
@@ -50,6 +56,9 @@ namespace ns {
 namespace {
 
 constexpr int kRowSlots = 4;                // slots per wave
+constexpr uint32_t kWideMaxWaves = 12;      // of a workgroup with one slot per wave
+constexpr uint32_t kSumCopies = 8;          // of a sum's words, one per XCD
+constexpr uint32_t kSumWords = kSumCopies * 256u * 4u;
 constexpr uint32_t kFaceFloats = 384;       // floats of a slot's six faces
 
 typedef unsigned v4u __attribute__((ext_vector_type(4)));
@@ -125,6 +134,40 @@ constexpr uint64_t plane_lanes(int m, int b, int k) {
     for (int l = 0; l < 16; ++l)
         if (((m - b - (l & 7) - 4 * (l >> 3)) & 7) == k) row |= 1u << l;
     return (uint64_t)(row | (row << 16)) * 0x100000001ull;
+}
+
+// One slot per wave: the lanes (8 j + i) with a cell of step t, and those whose
+// register m holds plane k.
+constexpr uint64_t wide_lanes(int t) {
+    uint64_t o = 0;
+    for (int l = 0; l < 64; ++l) {
+        const int k = t - (l & 7) - (l >> 3);
+        if (k >= 0 && k <= 7) o |= 1ull << l;
+    }
+    return o;
+}
+constexpr uint64_t wide_plane(int m, int k) {
+    uint64_t o = 0;
+    for (int l = 0; l < 64; ++l)
+        if (((m - (l & 7) - (l >> 3)) & 7) == k) o |= 1ull << l;
+    return o;
+}
+// The value of the lane 8 below / above (any in the lanes that have none).
+// Half a row's neighbours are in its other half; the others come from the
+// next row: rows are exchanged by the swaps of 16 and of 32 lanes.
+__device__ inline float lane_up8(float v) {
+    const unsigned u = (unsigned)__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x128, 0xf, 0xf, true);  // halves swapped
+    const auto s16 = __builtin_amdgcn_permlane16_swap(u, u, false, false);            // rows 0 0 2 2, 1 1 3 3
+    const auto s32 = __builtin_amdgcn_permlane32_swap(s16[0], s16[1], false, false);  // rows 0 0 1 1, 2 2 3 3
+    const float low = lanes_or(0xffff000000000000ull, __uint_as_float(s16[0]), __uint_as_float(s32[0]));
+    return row_shift_or<kRowShr8, 0xc>(low, v);
+}
+__device__ inline float lane_down8(float v) {
+    const unsigned u = (unsigned)__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x128, 0xf, 0xf, true);
+    const auto s16 = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+    const auto s32 = __builtin_amdgcn_permlane32_swap(s16[0], s16[1], false, false);
+    const float high = lanes_or(0x000000000000ffffull, __uint_as_float(s16[1]), __uint_as_float(s32[1]));
+    return row_shift_or<kRowShl8, 0x3>(high, v);
 }
 
 // Forward and backward sweep of the MIC(0) factors pc: z = M^-1 z in place.
@@ -222,22 +265,23 @@ __device__ inline void wave_lds_order() {
 
 // What the workgroup shares besides e and the faces.
 struct Shared {
-    double slot[2][4 * kResidentMaxWaves];  // per-slot sums
+    double slot[2][4 * kWideMaxWaves];  // per-slot sums
     double part[2][16];                     // row sums of the published values
     uint32_t bad;
 };
 
-// Grid-wide sums of a and (N == 2) c.  Words: N * 2 per workgroup at words.
+// Grid-wide sums of a and (N == 2) b.  Words: N * 2 of 4 per workgroup and copy.
 // False when a wait ran out.  Every thread of every workgroup gets the sums.
 template <int N>
-__device__ inline bool grid_sum(Shared& sh, double a, double c, uint64_t* words, uint32_t number, uint32_t groups,
-                                uint32_t polls, double& sa, double& sc) {
+__device__ inline bool grid_sum(Shared& sh, double a, double b, const CgResident& c, uint64_t* words,
+                                uint32_t number, double& sa, double& sb) {
+    const uint32_t groups = c.groups;
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6, waves = blockDim.x >> 6;
     a = row_sum(a);
-    if (N == 2) c = row_sum(c);
+    if (N == 2) b = row_sum(b);
     if ((lane & 15u) == 15u) {
         sh.slot[0][wave * 4u + (lane >> 4)] = a;
-        if (N == 2) sh.slot[1][wave * 4u + (lane >> 4)] = c;
+        if (N == 2) sh.slot[1][wave * 4u + (lane >> 4)] = b;
     }
     // the faces written before this sum are in memory before it is announced
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -254,7 +298,9 @@ __device__ inline bool grid_sum(Shared& sh, double a, double c, uint64_t* words,
             if (N == 2) ty += lane_value(y, 16 * r + 15);
         }
         if (groups > 1u) {
-            if (lane < 2u * N) publish(words + blockIdx.x * 2u * N + lane, lane < 2u ? tx : ty, (int)(lane & 1u), number);
+            const uint32_t copy = lane / (2u * N), q = lane % (2u * N);
+            if (copy < kSumCopies)
+                publish(words + (copy * 256u + blockIdx.x) * 4u + q, q < 2u ? tx : ty, (int)(q & 1u), number);
         } else if (lane == 0) {
             sh.part[0][0] = tx;
             if (N == 2) sh.part[1][0] = ty;
@@ -264,10 +310,11 @@ __device__ inline bool grid_sum(Shared& sh, double a, double c, uint64_t* words,
         if (tid < 256u) {
             double x = 0.0, y = 0.0;
             if (tid < groups) {
-                const uint64_t* w = words + tid * 2u * N;
+                const uint64_t* w = words + ((blockIdx.x & (kSumCopies - 1u)) * 256u + tid) * 4u;
                 uint64_t v[2 * N] = {};
+                for (uint32_t t = 0; t < c.pause; ++t) __builtin_amdgcn_s_sleep(1);
                 for (uint32_t poll = 0;; ++poll) {
-                    if (poll >= polls) {
+                    if (poll >= c.polls) {
                         sh.bad = 1u;
                         break;
                     }
@@ -292,16 +339,16 @@ __device__ inline bool grid_sum(Shared& sh, double a, double c, uint64_t* words,
         __syncthreads();
         if (sh.bad) return false;
         sa = sh.part[0][0];
-        if (N == 2) sc = sh.part[1][0];
+        if (N == 2) sb = sh.part[1][0];
         const uint32_t rows = (groups + 15u) >> 4;
         for (uint32_t r = 1; r < rows; ++r) {
             sa += sh.part[0][r];
-            if (N == 2) sc += sh.part[1][r];
+            if (N == 2) sb += sh.part[1][r];
         }
     } else {
         __syncthreads();
         sa = sh.part[0][0];
-        if (N == 2) sc = sh.part[1][0];
+        if (N == 2) sb = sh.part[1][0];
     }
     return true;
 }
@@ -312,6 +359,7 @@ __device__ inline bool grid_sum(Shared& sh, double a, double c, uint64_t* words,
 // p (6 x 64 float4: -x, +x, y in two halves, -z, +z), laid out as a lane
 // loads them.
 constexpr uint32_t kWaveLds = (8u + 6u) * 64u * 16u;
+constexpr uint32_t kWideLds = 80u * 32u;  // one slot per wave: p of its rows j = -1 .. 8
 
 template <int MIC, int WAVES>
 __global__ void __launch_bounds__(64 * WAVES)
@@ -452,7 +500,7 @@ pcg_resident_kernel(CgResident c) {
                 srr += (double)r[b][m] * (double)r[b][m];
             }
         double rz, rr;
-        if (!grid_sum<2>(sh, srz, srr, words, c.number + 2u * it, c.groups, c.polls, rz, rr)) {
+        if (!grid_sum<2>(sh, srz, srr, c, words, c.number + 2u * it, rz, rr)) {
             failed = true;
             break;
         }
@@ -516,8 +564,7 @@ pcg_resident_kernel(CgResident c) {
             }
         }
         double pq, unused;
-        if (!grid_sum<1>(sh, spq, 0.0, words + 4u * c.groups, c.number + 2u * it + 1u, c.groups, c.polls, pq,
-                         unused)) {
+        if (!grid_sum<1>(sh, spq, 0.0, c, words + kSumWords, c.number + 2u * it + 1u, pq, unused)) {
             failed = true;
             break;
         }
@@ -559,14 +606,214 @@ pcg_resident_kernel(CgResident c) {
     }
 }
 
+// One slot per wave, for systems that leave the chip idle with four: lane
+// 8 j + i holds the column (i, j) of its slot, register m its k = (m - i - j)
+// mod 8 (as above, neighbours are at fixed registers; lanes 8 apart are
+// exchanged by row swaps in the sweeps and through LDS in the product), and
+// the correction e stays in registers.  A quarter of the instructions per
+// wave: 160 slots, Jacobi 6.5 -> 5.2 us per iteration, MIC(0) 9.1 -> 7.6
+// (before the sums' copies and pauses).
+template <int MIC>
+__global__ void __launch_bounds__(64 * kWideMaxWaves)
+pcg_wide_kernel(CgResident c) {
+    extern __shared__ __align__(16) unsigned char s_raw[];
+    Shared& sh = *reinterpret_cast<Shared*>(s_raw);
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
+    // p of rows j = -1 .. 8 (8 lanes of 8 registers each)
+    float4* s_p = reinterpret_cast<float4*>(s_raw + ((sizeof(Shared) + 15u) & ~15u) + wave * kWideLds) + 16 + 2 * lane;
+    const uint32_t i = lane & 7u, j = lane >> 3;
+    const int d0 = (int)(i + j);
+    const uint32_t slotRaw = blockIdx.x * waves + wave;
+    const bool live = slotRaw < c.na;
+    const uint32_t slot = live ? slotRaw : 0u;
+    const float in0 = i == 0u ? 0.f : 1.f, in7 = i == 7u ? 0.f : 1.f;
+    const float jn0 = j == 0u ? 0.f : 1.f, jn7 = j == 7u ? 0.f : 1.f;
+    if (threadIdx.x == 0) sh.bad = 0u;
+
+    const uint32_t base = slot * 512u + lane;
+    float r[8], p[8], pc[8], z[8], e[8], dg[8];
+    float xh[8], yh[8], zl = 0.f, zh = 0.f;  // the neighbours' faces of p (x: lanes i = 0, 7; y: j = 0, 7)
+    {
+        uint32_t cf[8];
+        double r0[8];
+        float f[8];
+#pragma unroll
+        for (int m = 0; m < 8; ++m) {
+            const uint32_t v = base + 64u * (uint32_t)((m - d0) & 7);
+            cf[m] = c.coef[v];
+            r0[m] = c.r64[v];
+            f[m] = MIC ? c.precon[v] : 0.f;
+        }
+#pragma unroll
+        for (int m = 0; m < 8; ++m) {
+            const uint32_t keep = live && cf[m] != 0u ? 0xffffffffu : 0u, diag = cf[m] & keep & 7u;
+            dg[m] = (float)diag;
+            if (!MIC) f[m] = 1.f / (float)max(diag, 1u);
+            r[m] = __uint_as_float(__float_as_uint((float)r0[m]) & keep);
+            pc[m] = __uint_as_float(__float_as_uint(f[m]) & keep);
+            p[m] = e[m] = xh[m] = yh[m] = 0.f;
+        }
+    }
+
+    constexpr uint32_t kNone = 0x80000000u;
+    const __amdgpu_buffer_rsrc_t faces =
+        __builtin_amdgcn_make_buffer_rsrc(c.faces, 0, c.na * kFaceFloats * 4u, 0x00027000);
+    // x faces [j][m], y faces [i][m] in the owner's register order, z faces [j][i]
+    const uint32_t mine = live ? slot * (kFaceFloats * 4u) : kNone;
+    const uint32_t outX = i == 0u ? mine + 32u * j : i == 7u ? mine + 256u + 32u * j : kNone;
+    const uint32_t outY = j == 0u ? mine + 512u + 32u * i : j == 7u ? mine + 768u + 32u * i : kNone;
+    const uint32_t outZ = mine + 1024u + 4u * lane;
+    auto nbr = [&](uint32_t d, uint32_t face, uint32_t add) {
+        const int32_t s = live ? c.nbrSlot[slot * 6u + d] : -1;
+        return s < 0 ? kNone : (uint32_t)s * (kFaceFloats * 4u) + 256u * face + add;
+    };
+    const uint32_t inX = i == 0u ? nbr(0, 1, 32u * j) : i == 7u ? nbr(1, 0, 32u * j) : kNone;
+    const uint32_t inY = j == 0u ? nbr(2, 3, 32u * i) : j == 7u ? nbr(3, 2, 32u * i) : kNone;
+    const uint32_t inZ0 = nbr(4, 5, 4u * lane), inZ1 = nbr(5, 4, 4u * lane);
+
+    uint64_t* words = c.words;
+    double rzOld = 0.0;
+    uint32_t it = 0;
+    bool failed = false;
+    for (;; ++it) {
+#pragma unroll
+        for (int m = 0; m < 8; ++m) {
+            z[m] = r[m];
+            if (!MIC) {
+                const float q = r[m] * pc[m];
+                z[m] = fmaf(fmaf(-q, dg[m], r[m]), pc[m], q);
+            }
+        }
+        if (MIC) {
+            float w = 0.f;
+#pragma unroll
+            for (int t = 0; t < 22; ++t) {
+                const int m = t & 7;
+                float acc = z[m] + w;
+                acc = fmaf(row_shift<kRowShr1>(w), in0, acc);
+                acc = fmaf(lane_up8(w), jn0, acc);
+                const float q = acc * pc[m];
+                z[m] = lanes_or(wide_lanes(t), q, z[m]);
+                w = lanes_or(wide_lanes(t), q * pc[m], 0.f);
+            }
+            float u = 0.f;
+#pragma unroll
+            for (int t = 21; t >= 0; --t) {
+                const int m = t & 7;
+                const float f = pc[m];
+                float acc = fmaf(f, u, z[m]);
+                acc = fmaf(f, row_shift<kRowShl1>(u) * in7, acc);
+                acc = fmaf(f, lane_down8(u) * jn7, acc);
+                const float x = acc * f;
+                z[m] = lanes_or(wide_lanes(t), x, z[m]);
+                u = lanes_or(wide_lanes(t), x, 0.f);
+            }
+        }
+        __builtin_amdgcn_raw_buffer_store_b128(pack4(z[0], z[1], z[2], z[3]), faces, outX, 0, kAgent);
+        __builtin_amdgcn_raw_buffer_store_b128(pack4(z[4], z[5], z[6], z[7]), faces, outX + 16u, 0, kAgent);
+        __builtin_amdgcn_raw_buffer_store_b128(pack4(z[0], z[1], z[2], z[3]), faces, outY, 0, kAgent);
+        __builtin_amdgcn_raw_buffer_store_b128(pack4(z[4], z[5], z[6], z[7]), faces, outY + 16u, 0, kAgent);
+        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(plane_value<0>(z, 0, d0)), faces, outZ, 0, kAgent);
+        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(plane_value<7>(z, 0, d0)), faces, outZ + 256u, 0, kAgent);
+        double srz = 0.0, srr = 0.0;
+#pragma unroll
+        for (int m = 0; m < 8; ++m) {
+            srz += (double)r[m] * (double)z[m];
+            srr += (double)r[m] * (double)r[m];
+        }
+        double rz, rr;
+        if (!grid_sum<2>(sh, srz, srr, c, words, c.number + 2u * it, rz, rr)) {
+            failed = true;
+            break;
+        }
+        if (rr <= c.thr2 || !(rr == rr) || it == c.limit) break;  // the same decision everywhere
+        const float beta = it == 0u ? 0.f : rzOld != 0.0 ? (float)(rz / rzOld) : 0.f;
+        rzOld = rz;
+        v4u h4[4];
+        uint32_t h1[2];
+        h4[0] = __builtin_amdgcn_raw_buffer_load_b128(faces, inX, 0, kAgent);
+        h4[1] = __builtin_amdgcn_raw_buffer_load_b128(faces, inX + 16u, 0, kAgent);
+        h4[2] = __builtin_amdgcn_raw_buffer_load_b128(faces, inY, 0, kAgent);
+        h4[3] = __builtin_amdgcn_raw_buffer_load_b128(faces, inY + 16u, 0, kAgent);
+        h1[0] = __builtin_amdgcn_raw_buffer_load_b32(faces, inZ0, 0, kAgent);
+        h1[1] = __builtin_amdgcn_raw_buffer_load_b32(faces, inZ1, 0, kAgent);
+#pragma unroll
+        for (int m = 0; m < 8; ++m) p[m] = fmaf(beta, p[m], z[m]);
+        s_p[0] = make_float4(p[0], p[1], p[2], p[3]);
+        s_p[1] = make_float4(p[4], p[5], p[6], p[7]);
+#pragma unroll
+        for (int m = 0; m < 8; ++m) {
+            const v4u hx = h4[m >> 2], hy = h4[2 + (m >> 2)];
+            xh[m] = fmaf(beta, xh[m], __uint_as_float(hx[m & 3]));
+            yh[m] = fmaf(beta, yh[m], __uint_as_float(hy[m & 3]));
+        }
+        zl = fmaf(beta, zl, __uint_as_float(h1[0]));
+        zh = fmaf(beta, zh, __uint_as_float(h1[1]));
+        if (j == 0u || j == 7u) {
+            float4* o = s_p + (j == 0u ? -16 : 16);
+            o[0] = make_float4(yh[0], yh[1], yh[2], yh[3]);
+            o[1] = make_float4(yh[4], yh[5], yh[6], yh[7]);
+        }
+        wave_lds_order();
+        const float4 a0 = s_p[-16], a1 = s_p[-15], b0 = s_p[16], b1 = s_p[17];
+        const float ym[8] = {a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w};
+        const float yp[8] = {b0.x, b0.y, b0.z, b0.w, b1.x, b1.y, b1.z, b1.w};
+        double spq = 0.0;
+        float q[8];
+#pragma unroll
+        for (int m = 0; m < 8; ++m) {
+            const int lo = (m + 7) & 7, hi = (m + 1) & 7;
+            float s = dg[m] * p[m];
+            s -= lanes_or(0x0101010101010101ull, xh[lo], row_shift<kRowShr1>(p[lo]));
+            s -= lanes_or(0x8080808080808080ull, xh[hi], row_shift<kRowShl1>(p[hi]));
+            s -= ym[lo];
+            s -= yp[hi];
+            s -= lanes_or(wide_plane(m, 0), zl, p[lo]);
+            s -= lanes_or(wide_plane(m, 7), zh, p[hi]);
+            q[m] = pc[m] != 0.f ? s : 0.f;
+            spq += (double)p[m] * (double)q[m];
+        }
+        wave_lds_order();  // the next iteration's writes come after these reads
+        double pq, unused;
+        if (!grid_sum<1>(sh, spq, 0.0, c, words + kSumWords, c.number + 2u * it + 1u, pq, unused)) {
+            failed = true;
+            break;
+        }
+        const float alpha = pq != 0.0 ? (float)(rz / pq) : 0.f;
+#pragma unroll
+        for (int m = 0; m < 8; ++m) {
+            e[m] = fmaf(alpha, p[m], e[m]);
+            r[m] = fmaf(-alpha, q[m], r[m]);
+        }
+    }
+
+    if (!failed && live) {
+        double x[8];
+#pragma unroll
+        for (int m = 0; m < 8; ++m) x[m] = c.x64[base + 64u * (uint32_t)((m - d0) & 7)];
+#pragma unroll
+        for (int m = 0; m < 8; ++m)
+            if (pc[m] != 0.f) c.x64[base + 64u * (uint32_t)((m - d0) & 7)] = x[m] + (double)e[m];
+    }
+    if (threadIdx.x == 0) {
+        if (blockIdx.x == 0) c.result[0] = it;
+        if (failed) c.result[1] = c.number;
+    }
+}
+
 namespace {
-// Up to eight waves (two per SIMD) a lane may use 256 registers, above 168.
 using ResidentKernel = void (*)(CgResident);
-ResidentKernel resident_kernel(bool mic, uint32_t waves) {
-    if (waves <= 8u) return mic ? pcg_resident_kernel<1, 8> : pcg_resident_kernel<0, 8>;
+ResidentKernel resident_kernel(bool mic, const ResidentShape& s) {
+    if (s.wide) {
+        return mic ? pcg_wide_kernel<1> : pcg_wide_kernel<0>;
+    }
+    // up to eight waves (two per SIMD) a lane may use 256 registers, above 168
+    if (s.waves <= 8u) return mic ? pcg_resident_kernel<1, 8> : pcg_resident_kernel<0, 8>;
     return mic ? pcg_resident_kernel<1, kResidentMaxWaves> : pcg_resident_kernel<0, kResidentMaxWaves>;
 }
-size_t resident_lds(uint32_t waves) { return ((sizeof(Shared) + 15u) & ~(size_t)15u) + (size_t)waves * kWaveLds; }
+size_t resident_lds(const ResidentShape& s) {
+    return ((sizeof(Shared) + 15u) & ~(size_t)15u) + (size_t)s.waves * (s.wide ? kWideLds : kWaveLds);
+}
 }  // namespace
 
 ResidentShape resident_shape(uint32_t na, bool mic) {
@@ -576,21 +823,27 @@ ResidentShape resident_shape(uint32_t na, bool mic) {
     FLIP2_HIP(hipGetDevice(&dev));
     FLIP2_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
     FLIP2_HIP(hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev));
-    const uint32_t all = ceil_div(na, kRowSlots);
     const uint32_t most = std::min<uint32_t>(256u, (uint32_t)cus);
-    // one wave per SIMD as long as the CUs suffice (an iteration of a wave is
-    // a chain of instructions; the fewest workgroups have the fewest sums)
-    const uint32_t waves = std::max(4u, ceil_div(all, most));
-    if (waves > (uint32_t)kResidentMaxWaves || resident_lds(waves) > (size_t)lds) return s;
-    s.groups = ceil_div(all, waves);
-    s.waves = waves;
+    // One slot per wave as long as the CUs hold the waves with the registers
+    // they need (per iteration, four slots per wave -> one: 960 slots Jacobi
+    // 7.3 -> 5.5 us, 1370 slots 7.3 -> 5.9 and MIC(0) 10.2 -> 9.2, 2508 slots
+    // Jacobi 8.0 -> 7.4).  With MIC(0) only up to two waves per SIMD: beyond,
+    // its sweeps, which keep four columns per lane busy in the other layout
+    // and one here, are bound by instruction issue (2383 slots 9.8 against
+    // 10.3 us).  At least four waves, one per SIMD: an iteration of a wave is
+    // a chain of instructions, and fewer workgroups have fewer sums.
+    s.wide = na <= (mic ? 8u : kWideMaxWaves) * most;
+    const uint32_t all = s.wide ? na : ceil_div(na, kRowSlots);
+    s.waves = std::max(4u, ceil_div(all, most));
+    if ((!s.wide && s.waves > (uint32_t)kResidentMaxWaves) || resident_lds(s) > (size_t)lds) return s;
     int per = 0;
-    FLIP2_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, resident_kernel(mic, waves), 64 * (int)waves,
-                                                           resident_lds(waves)));
-    if (per < 1) s.groups = 0;
+    FLIP2_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, resident_kernel(mic, s), 64 * (int)s.waves,
+                                                           resident_lds(s)));
+    if (per >= 1) s.groups = ceil_div(all, s.waves);
     return s;
 }
 
+size_t resident_words() { return 2u * kSumWords; }
 size_t resident_face_floats(uint32_t na) { return (size_t)na * kFaceFloats; }
 
 std::mutex& resident_mutex(int device) {
@@ -600,11 +853,20 @@ std::mutex& resident_mutex(int device) {
 
 void launch_pcg_resident(const CgResident& c, const ResidentShape& shape, bool mic, hipStream_t s) {
     FLIP2_REQUIRE(c.na && c.na <= (1u << 20) && shape.groups && c.groups == shape.groups && shape.groups <= 256u &&
-                      (uint64_t)shape.groups * shape.waves * kRowSlots >= c.na,
+                      (uint64_t)shape.groups * shape.waves * (shape.wide ? 1u : kRowSlots) >= c.na,
                   kErrArgument, "resident PCG: the grid does not hold the slots");
-    const size_t lds = resident_lds(shape.waves);
-    const ResidentKernel pcg_resident_kernel = resident_kernel(mic, shape.waves);
-    FLIP2_KERNEL(pcg_resident_kernel, dim3(shape.groups), dim3(64 * shape.waves), lds, s, c);
+    const size_t lds = resident_lds(shape);
+    const ResidentKernel pcg_resident_kernel = resident_kernel(mic, shape);
+    CgResident k = c;
+    // The words arrive after the latency of a write and a read.  Reads that
+    // come earlier find nothing and hold up the others' writes and faces, the
+    // more workgroups the worse; a pause that is too long is paid in full.
+    // Per iteration without / with a pause (64 clocks each): 12 slots 4.66 ->
+    // 4.58 us with 4 (5.25 with 18), 160 slots 4.70 -> 4.28 with 10 (4.69 with
+    // 18), 960 slots 7.72 -> 5.47 with 18 (5.96 with 10), 9196 slots MIC(0)
+    // 25.0 -> 22.7 with 40 (24.2 with 18).
+    k.pause = shape.groups <= 16u ? 4u : shape.groups <= 64u ? 10u : shape.waves <= 8u || shape.wide ? 18u : 36u;
+    FLIP2_KERNEL(pcg_resident_kernel, dim3(shape.groups), dim3(64 * shape.waves), lds, s, k);
     FLIP2_LAUNCH_CHECK();
 }
 

@@ -1,8 +1,9 @@
 """The resident PCG (one launch per refinement) against the two-kernel form
 (taken for iteration caps above 16384), on the same systems: one workgroup and
-several, rows of a wave and waves of a workgroup that hold no slot, one to
-three waves per SIMD and both register budgets, and one slot more than fits
-(both are then the two-kernel form).  Both solve to the same FP64 residual;
+several, one and four slots per wave around the sizes where the layout changes
+(2048 slots with MIC(0), 3072 with Jacobi), rows of a wave and waves of a
+workgroup that hold no slot, one to three waves per SIMD and both register
+budgets, and one slot more than fits (both are then the two-kernel form).  Both solve to the same FP64 residual;
 with the same rounding of every vector update they take the same iterations
 up to the last few, and their pressures differ by the solver's tolerance times
 a factor for the operator's condition, far below 1e-4."""
@@ -32,7 +33,7 @@ def _bricks(n, seed):
 
 
 @pytest.mark.parametrize("prec", ["jacobi", "mic0"])
-@pytest.mark.parametrize("n", [1, 4, 5, 16, 17, 63, 1000, 4096, 4101, 8192, 8195, 11264, 11265])
+@pytest.mark.parametrize("n", [1, 4, 5, 16, 17, 63, 1000, 1025, 2048, 2049, 3072, 3073, 4096, 4101, 8192, 8195, 11264, 11265])
 def test_resident_matches_two_kernel_form(flip2, n, prec):
     grid, pos, vel = _bricks(n, n)
     got = []
