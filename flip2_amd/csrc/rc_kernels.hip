@@ -429,105 +429,120 @@ __device__ inline bool is_apron(uint32_t id) {
     return x < 1u || x >= rb || y < 1u || y >= rb || z < 1u || z >= rb;
 }
 
-// isRed (voxelSolveFunctions.cu:286-291).
-__device__ inline bool is_red(uint32_t id) {
-    const uint32_t x = id % N1, y = (id % (N1 * N1)) / N1, z = id / (N1 * N1);
-    return !((x + y + z) & 1u);
-}
-
 }  // namespace
 
+// n / d, rounded as the quotient, with r = 1 / d rounded (d > 0): n r is
+// within two units of n / d, its correction within one, and the correction of
+// a value within one unit is the correctly rounded quotient where nothing
+// over- or underflows (Markstein 1990); the division itself elsewhere.  Five
+// instructions in a row against about ten of the division.
+__device__ inline double quotient(double n, double d, double r) {
+    const double q = n * r;
+    const double c = fma(fma(-q, d, n), r, q);
+    if (fabs(q) > 0x1p-900 && fabs(q) < 0x1p+900 && d < 0x1p+100 && d > 0x1p-100) return fma(fma(-c, d, n), r, c);
+    return n == 0.0 ? q : n / d;
+}
+
 // `iters` red/black iterations of GSiteration (voxelSolveFunctions.cu:293-389)
-// with the node tile resident in LDS.  Each thread owns voxel slots tid and
-// tid+256.  A half-sweep computes every new value from the tile as it was at
-// the start of the half-sweep, then stores them.  The residual written is the
-// one of the last (black) half-sweep: non-updated voxels hold 0.
-__global__ void __launch_bounds__(256)
+// with the node tile resident in LDS.  Updated are the voxels with x and z in
+// 1..6 (is_apron's "y" is x), 144 of each colour (isRed, voxelSolveFunctions.cu:286-291: x + y + z even): thread e < 144 owns the e-th
+// of both, so a half-sweep is three waves' work (with the voxels dealt by
+// list order it was eight, half of their lanes of the other colour).  What
+// bounds it: the chain of LDS reads, six products, quotient and two barriers
+// of a half-sweep, with the few workgroups that a CU holds (12 x 16 x 32
+// cells of particles, 64 iterations: 198 -> 172 us).  A
+// half-sweep computes every new value from the tile as it was at the start of
+// the half-sweep, then stores them (rows y = 0 and 7 read voxels of their own
+// colour).  The residual written is the one of the last (black) half-sweep:
+// non-updated voxels hold 0.
+constexpr uint32_t kSorThreads = 192;
+// The tile's voxels in LDS: rows 12 apart, so the 24 voxels (six x, four y)
+// of one colour and z are in different banks.
+__device__ inline uint32_t sor_index(uint32_t id) { return (id & 7u) + 12u * ((id >> 3) & 7u) + 96u * (id >> 6); }
+
+__global__ void __launch_bounds__(kSorThreads)
 sor_kernel(const uint32_t* __restrict__ nodeOff, const uint32_t* __restrict__ voxelIDs,
            const char* __restrict__ solids, const double* __restrict__ divU, double* __restrict__ p,
            double* __restrict__ residuals, double scale, double w, uint32_t iters) {
-    __shared__ double s_p[NV];
-    __shared__ double s_d[NV];
-    __shared__ uint8_t s_sol[NV];
+    static_assert(N1 == 8u, "sor_index");
+    __shared__ double s_p[768];
+    __shared__ double s_d[NV];  // divU, then the residuals
+    __shared__ uint8_t s_sol[NV], s_in[NV];
     const uint32_t b = blockIdx.x;
     const uint32_t tid = threadIdx.x;
-    for (uint32_t i = tid; i < NV; i += 256) { s_p[i] = 0.0; s_d[i] = 0.0; s_sol[i] = 0; }
+    for (uint32_t i = tid; i < NV; i += kSorThreads) { s_p[sor_index(i)] = 0.0; s_d[i] = 0.0; s_sol[i] = 0; s_in[i] = 0; }
     __syncthreads();
     const uint32_t vs = (b == 0) ? 0u : nodeOff[b - 1];
     const uint32_t cnt = nodeOff[b] - vs;
-    for (uint32_t k = tid; k < cnt; k += 256) {
+    for (uint32_t k = tid; k < cnt; k += kSorThreads) {
         const uint32_t id = voxelIDs[vs + k];
-        s_p[id] = p[vs + k];
+        s_p[sor_index(id)] = p[vs + k];
         s_d[id] = divU[vs + k];
         s_sol[id] = (uint8_t)solids[vs + k];
+        s_in[id] = 1;
     }
     __syncthreads();
 
-    // Per-slot coefficients (divU and solids are constant during the solve).
-    uint32_t id[2];
-    int colour[2];  // 1 red, 0 black, -1 not updated
-    double A[2][6], Adiag[2], dv[2], res[2];
+    // The coefficients of the thread's black (0) and red (1) voxel (divU and
+    // solids are constant during the solve).
+    uint32_t id[2], at[2], yLo[2], yHi[2];  // in the list's numbering; in s_p, with the neighbours in y
+    bool own[2];
+    double rd[2];  // 1 / the diagonal
+    double A[2][6], Adiag[2], dv[2], res = 0.0;
     const int32_t off[6] = {-1, 1, -(int32_t)N1, (int32_t)N1, -(int32_t)(N1 * N1), (int32_t)(N1 * N1)};
+    const uint32_t e = tid < 144u ? tid : 0u;
+    const uint32_t x = 1u + e % 6u, z = 1u + e / 24u;
 #pragma unroll
-    for (int s = 0; s < 2; ++s) {
-        const uint32_t k = tid + 256u * s;
-        colour[s] = -1;
-        id[s] = 0;
-        Adiag[s] = 0.0;
-        dv[s] = 0.0;
-        res[s] = 0.0;
-        for (int j = 0; j < 6; ++j) A[s][j] = 0.0;
-        if (k < cnt) {
-            const uint32_t v = voxelIDs[vs + k];
-            id[s] = v;
-            dv[s] = s_d[v];
-            if (!s_sol[v] && !is_apron(v)) {
-                colour[s] = is_red(v) ? 1 : 0;
-                double ad = 0.0;
-                for (int j = 0; j < 6; ++j) {
-                    const uint32_t nbv = (uint32_t)((int32_t)v + off[j]);
-                    if (!s_sol[nbv]) {
-                        if (s_d[nbv] != 0.0) A[s][j] = -scale;
-                        ad = ad + scale;
-                    }
-                }
-                Adiag[s] = ad;
+    for (int red = 0; red < 2; ++red) {
+        const uint32_t y = 2u * ((e / 6u) & 3u) + ((x + z + (red ? 0u : 1u)) & 1u);
+        const uint32_t v = x + N1 * y + N1 * N1 * z;
+        id[red] = v;
+        at[red] = sor_index(v);
+        yLo[red] = sor_index(v - N1);
+        yHi[red] = sor_index(v + N1);
+        own[red] = tid < 144u && s_in[v] && !s_sol[v];
+        Adiag[red] = 0.0;
+        dv[red] = s_d[v];
+#pragma unroll
+        for (int j = 0; j < 6; ++j) {
+            const uint32_t nbv = (uint32_t)((int32_t)v + off[j]);
+            A[red][j] = 0.0;
+            if (!s_sol[nbv]) {
+                if (s_d[nbv] != 0.0) A[red][j] = -scale;
+                Adiag[red] = Adiag[red] + scale;
             }
         }
+        rd[red] = 1.0 / (Adiag[red] + 0.000000001);
     }
+    __syncthreads();
+    for (uint32_t i = tid; i < NV; i += kSorThreads) s_d[i] = 0.0;
 
     for (uint32_t it = 0; it < iters; ++it) {
-        for (int red = 1; red >= 0; --red) {
-            double pn[2];
 #pragma unroll
-            for (int s = 0; s < 2; ++s) {
-                res[s] = 0.0;
-                pn[s] = 0.0;
-                if (colour[s] == red) {
-                    const uint32_t v = id[s];
-                    const double sum = A[s][0] * s_p[v - 1] + A[s][1] * s_p[v + 1] + A[s][2] * s_p[v - N1] +
-                                       A[s][3] * s_p[v + N1] + A[s][4] * s_p[v - N1 * N1] +
-                                       A[s][5] * s_p[v + N1 * N1];
-                    const double pv = s_p[v];
-                    const double dg = Adiag[s] + 0.000000001;
-                    const double q = pv + w * ((-dv[s] - sum) / dg - pv);
-                    pn[s] = q;
-                    res[s] = (-dv[s] - dg * q + sum);
-                }
+        for (int red = 1; red >= 0; --red) {
+            const uint32_t a = at[red];
+            double q = 0.0;
+            if (own[red]) {
+                const double sum = A[red][0] * s_p[a - 1] + A[red][1] * s_p[a + 1] + A[red][2] * s_p[yLo[red]] +
+                                   A[red][3] * s_p[yHi[red]] + A[red][4] * s_p[a - 96u] + A[red][5] * s_p[a + 96u];
+                const double pv = s_p[a];
+                const double dg = Adiag[red] + 0.000000001;
+                q = pv + w * (quotient(-dv[red] - sum, dg, rd[red]) - pv);
+                res = (-dv[red] - dg * q + sum);
             }
             __syncthreads();
-#pragma unroll
-            for (int s = 0; s < 2; ++s)
-                if (colour[s] == red) s_p[id[s]] = pn[s];
+            if (own[red]) s_p[a] = q;
             __syncthreads();
         }
     }
-    for (int s = 0; s < 2; ++s) {
-        const uint32_t k = tid + 256u * s;
-        if (k < cnt) {
-            p[vs + k] = s_p[id[s]];
-            if (iters) residuals[vs + k] = res[s];
-        }
+    if (iters) {
+        if (own[0]) s_d[id[0]] = res;
+        __syncthreads();
+    }
+    for (uint32_t k = tid; k < cnt; k += kSorThreads) {
+        const uint32_t v = voxelIDs[vs + k];
+        p[vs + k] = s_p[sor_index(v)];
+        if (iters) residuals[vs + k] = s_d[v];
     }
 }
 
@@ -596,9 +611,16 @@ velocity_update_kernel(const uint32_t* __restrict__ nodeOff, const uint32_t* __r
     }
 }
 
+constexpr uint32_t kG2pThreads = 192;
+
 // gatherVoxelVelsToParticles (particles.cu:562-662), three components.
-// Lane = particle; the stencil is summed in the reference's loop order.
-__global__ void __launch_bounds__(64)
+// Lane = one component of one particle; the stencil is summed in the
+// reference's loop order.  A sum is a serial chain of up to 64 FP64 distances
+// and weights, and a node's ~20 particles filled a third of one wave that
+// took the components in turn: three waves share the (component, particle)
+// pairs, and weights of absent velocities are not formed (12 x 16 x 32 cells of
+// particles: 224 -> 63 us).
+__global__ void __launch_bounds__(kG2pThreads)
 g2p_kernel(uint32_t B, uint32_t n, Grid g, const uint32_t* __restrict__ keys, const uint32_t* __restrict__ first,
            const double* __restrict__ px, const double* __restrict__ py, const double* __restrict__ pz,
            double* __restrict__ vx, double* __restrict__ vy, double* __restrict__ vz,
@@ -607,11 +629,11 @@ g2p_kernel(uint32_t B, uint32_t n, Grid g, const uint32_t* __restrict__ keys, co
     __shared__ double s_t[3][NV];
     const uint32_t b = blockIdx.x;
     const uint32_t lane = threadIdx.x;
-    for (uint32_t i = lane; i < NV; i += 64) { s_t[0][i] = 0.0; s_t[1][i] = 0.0; s_t[2][i] = 0.0; }
+    for (uint32_t i = lane; i < NV; i += kG2pThreads) { s_t[0][i] = 0.0; s_t[1][i] = 0.0; s_t[2][i] = 0.0; }
     __syncthreads();
     const uint32_t vs = (b == 0) ? 0u : nodeOff[b - 1];
     const uint32_t ve = nodeOff[b];
-    for (uint32_t k = vs + lane; k < ve; k += 64) {
+    for (uint32_t k = vs + lane; k < ve; k += kG2pThreads) {
         const uint32_t id = voxelIDs[k];
         s_t[0][id] = Ux[k]; s_t[1][id] = Uy[k]; s_t[2][id] = Uz[k];
     }
@@ -621,31 +643,28 @@ g2p_kernel(uint32_t B, uint32_t n, Grid g, const uint32_t* __restrict__ keys, co
     const double rs = kRcRadius * scw;
     const uint32_t last = node_last(first, b, B, n);
     double* vel[3] = {vx, vy, vz};
-    for (uint32_t idx = first[b] + lane; idx < last; idx += 64) {
+    const uint32_t begin = first[b], count = last - begin;
+    for (uint32_t t = lane; t < 3u * count; t += kG2pThreads) {
+        const uint32_t c = t / count, idx = begin + (t - c * count);
         const Frame f = make_frame(g, keys[idx], px[idx], py[idx], pz[idx]);
-        const bool runs = stencil_runs(f);
-        for (int c = 0; c < 3; ++c) {
-            double sx, sy, sz;
-            stagger(c, hs, sx, sy, sz);
-            double pv = 0.0, ws = 0.0;
-            if (runs) {
-                for (uint32_t x = f.sub[0] - kRcApron; x < N1 && x < f.sub[0] + kRcApron; ++x)
-                    for (uint32_t y = f.sub[1] - kRcApron; y < N1 && y < f.sub[1] + kRcApron; ++y)
-                        for (uint32_t z = f.sub[2] - kRcApron; z < N1 && z < f.sub[2] + kRcApron; ++z) {
-                            const double bx = (double)(int32_t)x * scw + sx;
-                            const double by = (double)(int32_t)y * scw + sy;
-                            const double bz = (double)(int32_t)z * scw + sz;
-                            const double wt =
-                                ref_weight(ref_distance(f.pin[0] - bx, f.pin[1] - by, f.pin[2] - bz), rs);
-                            const double u = s_t[c][x + y * N1 + z * N1 * N1];
-                            if (u != 0.0) {
-                                ws = ws + wt;
-                                pv = pv + wt * u;
-                            }
-                        }
-            }
-            vel[c][idx] = pv / (ws + 0.00000001);
+        double sx, sy, sz;
+        stagger((int)c, hs, sx, sy, sz);
+        double pv = 0.0, ws = 0.0;
+        if (stencil_runs(f)) {
+            for (uint32_t x = f.sub[0] - kRcApron; x < N1 && x < f.sub[0] + kRcApron; ++x)
+                for (uint32_t y = f.sub[1] - kRcApron; y < N1 && y < f.sub[1] + kRcApron; ++y)
+                    for (uint32_t z = f.sub[2] - kRcApron; z < N1 && z < f.sub[2] + kRcApron; ++z) {
+                        const double u = s_t[c][x + y * N1 + z * N1 * N1];
+                        if (u == 0.0) continue;
+                        const double bx = (double)(int32_t)x * scw + sx;
+                        const double by = (double)(int32_t)y * scw + sy;
+                        const double bz = (double)(int32_t)z * scw + sz;
+                        const double wt = ref_weight(ref_distance(f.pin[0] - bx, f.pin[1] - by, f.pin[2] - bz), rs);
+                        ws = ws + wt;
+                        pv = pv + wt * u;
+                    }
         }
+        vel[c][idx] = pv / (ws + 0.00000001);
     }
 }
 
@@ -823,7 +842,7 @@ void launch_sor(uint32_t B, const uint32_t* nodeOff, const uint32_t* voxelIDs, c
                 const double* divU, double* p, double* residuals, double scale, double w, uint32_t iters,
                 hipStream_t s) {
     if (!B) return;
-    FLIP2_KERNEL(sor_kernel, dim3(B), dim3(256), 0, s, nodeOff, voxelIDs, solids, divU, p, residuals, scale,
+    FLIP2_KERNEL(sor_kernel, dim3(B), dim3(kSorThreads), 0, s, nodeOff, voxelIDs, solids, divU, p, residuals, scale,
                        w, iters);
     FLIP2_LAUNCH_CHECK();
 }
@@ -850,7 +869,7 @@ void launch_g2p(uint32_t B, uint32_t n, Grid g, const uint32_t* keys, const uint
                 const double* py, const double* pz, double* vx, double* vy, double* vz, const uint32_t* nodeOff,
                 const uint32_t* voxelIDs, const double* Ux, const double* Uy, const double* Uz, hipStream_t s) {
     if (!B) return;
-    FLIP2_KERNEL(g2p_kernel, dim3(B), dim3(64), 0, s, B, n, g, keys, first, px, py, pz, vx, vy, vz, nodeOff,
+    FLIP2_KERNEL(g2p_kernel, dim3(B), dim3(kG2pThreads), 0, s, B, n, g, keys, first, px, py, pz, vx, vy, vz, nodeOff,
                        voxelIDs, Ux, Uy, Uz);
     FLIP2_LAUNCH_CHECK();
 }
