@@ -188,6 +188,7 @@ def _declare(l: ctypes.CDLL) -> None:
         "flip2_fluid_stage": [_vp, ctypes.c_char_p],
         "flip2_fluid_solve_with": [_vp, ctypes.c_int, ctypes.POINTER(SolveStatsC)],
         "flip2_fluid_last_solve": [_vp, ctypes.POINTER(SolveStatsC)],
+        "flip2_fluid_solve_form": [_vp, ctypes.POINTER(_u32), ctypes.POINTER(_u32)],
         "flip2_fluid_get_array": [_vp, ctypes.c_char_p, _vp, _sz, ctypes.POINTER(_sz)],
         "flip2_p2g_pipeline_timing": [_vp, ctypes.c_int, ctypes.c_char_p, _sz, ctypes.POINTER(_f64),
                                       ctypes.POINTER(ctypes.c_int)],
@@ -578,6 +579,14 @@ class FluidSim:
         s = SolveStatsC()
         check(lib().flip2_fluid_last_solve(self._h, ctypes.byref(s)))
         return _stats_dict(s)
+
+    def solve_form(self) -> dict:
+        """How the last solve ran: "resident_refinements", those of its
+        refinements that were one resident launch, and "give_ups", this
+        simulation's solves so far whose resident attempt was given up."""
+        r, g = ctypes.c_uint32(), ctypes.c_uint32()
+        check(lib().flip2_fluid_solve_form(self._h, ctypes.byref(r), ctypes.byref(g)))
+        return {"resident_refinements": int(r.value), "give_ups": int(g.value)}
 
     def set_unet(self, net: Optional[UNet], fallback_iterations: int = 0) -> None:
         """Attach `net` as the "learned" preconditioner (None detaches)."""

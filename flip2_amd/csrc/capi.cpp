@@ -847,6 +847,13 @@ int flip2_fluid_last_solve(flip2_fluid* f, flip2_solve_stats* stats) {
         to_stats(f->impl.lastSolve(), stats);
     });
 }
+int flip2_fluid_solve_form(flip2_fluid* f, uint32_t* resident_refinements, uint32_t* give_ups) {
+    return guarded([&] {
+        NEED(f);
+        if (resident_refinements) *resident_refinements = f->impl.lastSolve().residentRefinements;
+        if (give_ups) *give_ups = f->impl.residentGiveUps();
+    });
+}
 int flip2_fluid_get_array(flip2_fluid* f, const char* name, void* host, size_t capacity, size_t* count) {
     return guarded([&] {
         NEED(f); NEED(name);

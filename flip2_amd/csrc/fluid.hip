@@ -657,11 +657,12 @@ SolveStats FluidSim::solveOnce(int prec, uint32_t capIn) {
             ResidentEnd end = residentRefinement(na, shape, !jac, r64, thr * thr, cap - total);
             if (end.failed) {  // x64 is not usable: solve again without it
                 residentOk_ = false;
+                ++residentGiveUps_;
                 return solveOnce(prec, capIn);
             }
             total += end.iterations;
             rel = std::sqrt(std::max(end.rr, 0.0)) / st.bNorm;
-            st.refinements = refine + 1;
+            st.refinements = st.residentRefinements = refine + 1;
             if (rel <= cfg_.tolerance) {
                 st.converged = true;
                 break;

@@ -65,6 +65,7 @@ struct SolveStats {
     double solveMs = 0.0;          // wall time of the solve (host clock, synchronised)
     bool converged = false;
     bool usedFallback = false;
+    uint32_t residentRefinements = 0;  // of the refinements, those that were one resident launch
 };
 
 // A preconditioner supplied from outside the solver (the learned one):
@@ -146,6 +147,8 @@ public:
     // it is given up (the solve then runs again in the two-kernel form).
     void setResidentPolls(uint32_t polls) { residentPolls_ = polls; }
     bool residentUsable() const { return residentOk_; }
+    // Solves of this simulation whose resident attempt was given up.
+    uint32_t residentGiveUps() const { return residentGiveUps_; }
 
     const SolveStats& lastSolve() const { return stats_; }
     uint32_t numParticles() const { return n_; }
@@ -242,7 +245,7 @@ private:
     };
     ResidentEnd residentRefinement(uint32_t na, const ns::ResidentShape& shape, bool mic, const double* r64,
                                    double thr2, uint32_t limit);
-    uint32_t residentNumber_ = 0, residentPolls_ = ns::kResidentPolls;
+    uint32_t residentNumber_ = 0, residentPolls_ = ns::kResidentPolls, residentGiveUps_ = 0;
     bool residentOk_ = true;
     DeviceVec<uint32_t> total_{dm_};
     DeviceVec<uint8_t> ws_{dm_};

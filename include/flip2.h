@@ -346,6 +346,17 @@ int flip2_fluid_stage(flip2_fluid* f, const char* stage);
  * have been built by the "system" stage). */
 int flip2_fluid_solve_with(flip2_fluid* f, int preconditioner, flip2_solve_stats* stats);
 int flip2_fluid_last_solve(flip2_fluid* f, flip2_solve_stats* stats);
+/* The form in which the last solve ran.  A Jacobi- or MIC(0)-PCG whose active
+ * bricks fit the chip (up to 11264 on a whole MI355X) runs each refinement as
+ * one resident launch; two kernels per iteration serve larger systems,
+ * iteration caps above 16384, residual capture, and solves whose resident
+ * launch was given up (its workgroups wait for each other, and another
+ * process held the GPU's compute units for ~0.2 s).  *resident_refinements:
+ * refinements of the last solve that were one resident launch (0: the other
+ * form, or the learned preconditioner).  *give_ups: solves of this simulation
+ * so far whose resident attempt was given up.  Either may be NULL.  No
+ * counterpart in the reference. */
+int flip2_fluid_solve_form(flip2_fluid* f, uint32_t* resident_refinements, uint32_t* give_ups);
 /* "U","V","W","U0","V0","W0","counts","cellStart","activeBricks","brickSlot",
  * "cellType","coef","b","p". */
 int flip2_fluid_get_array(flip2_fluid* f, const char* name, void* host, size_t capacity, size_t* count);

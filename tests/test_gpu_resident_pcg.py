@@ -1,16 +1,19 @@
 """The resident PCG (one launch per refinement) against the two-kernel form
-(taken for iteration caps above 16384), on the same systems: one workgroup and
-several, one and four slots per wave around the sizes where the layout changes
-(2048 slots with MIC(0), 3072 with Jacobi), rows of a wave and waves of a
-workgroup that hold no slot, one to three waves per SIMD and both register
-budgets, and one slot more than fits (both are then the two-kernel form).  Both solve to the same FP64 residual;
-with the same rounding of every vector update they take the same iterations
-up to the last few, and their pressures differ by the solver's tolerance times
-a factor for the operator's condition, far below 1e-4."""
+(taken for iteration caps above 16384), on the same systems, each side in the
+form that its size and cap ask for: one workgroup and several, one and four
+slots per wave around the sizes where the layout changes (2048 slots with
+MIC(0), 3072 with Jacobi), rows of a wave and waves of a workgroup that hold
+no slot, one to three waves per SIMD and both register budgets, and one slot
+more than fits (both are then the two-kernel form).  Both solve to the same
+FP64 residual; with the same rounding of every vector update they take the
+same iterations up to the last few, and their pressures differ by the solver's
+tolerance times a factor for the operator's condition, far below 1e-4."""
 import numpy as np
 import pytest
 
 pytestmark = pytest.mark.gpu
+
+MOST = 11264  # slots that fit the chip: 256 CUs, eleven waves of four slots
 
 
 def _bricks(n, seed):
@@ -43,8 +46,12 @@ def test_resident_matches_two_kernel_form(flip2, n, prec):
         print(f"resident PCG: {n} bricks, {prec}, cap {cap}", flush=True)
         for stage in ("transfer_prepare", "system"):
             sim.stage(stage)
+        resident = n <= MOST and cap == 4000
         s = sim.solve_with(prec)
+        form = sim.solve_form()
+        assert form == {"resident_refinements": s["refinements"] if resident else 0, "give_ups": 0}, form
         again = sim.solve_with(prec)
+        assert sim.solve_form() == form
         assert s["active_bricks"] == n and s["converged"] and s["rel_residual"] <= 1e-6
         assert again["iterations"] == s["iterations"] and again["rel_residual"] == s["rel_residual"]  # deterministic
         got.append((s, sim.get("p")))
@@ -66,6 +73,7 @@ def test_resident_iteration_cap(flip2, prec):
         for stage in ("transfer_prepare", "system"):
             sim.stage(stage)
         got.append(sim.solve_with(prec))
+        assert (sim.solve_form()["resident_refinements"] > 0) == (cap == 7)
         sim.close()
     assert got[0]["iterations"] == 7 and not got[0]["converged"]
     assert got[1]["converged"] and got[1]["iterations"] > 7
