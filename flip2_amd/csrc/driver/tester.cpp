@@ -306,6 +306,38 @@ void run_resident_fallback() {
         sim.getArray("p", p[mode].data(), p[mode].size());
     }
     check(p[0] == p[1], "resident fallback: pressure");
+
+    // the rest after a give-up (16 solves), twice as long after another one in
+    // a row, and the resident form again once its waits end
+    FluidSim sim((uint32_t)x.size(), cfg);
+    sim.setParticles((uint32_t)x.size(), x.data(), y.data(), z.data(), v.data(), zero.data(), zero.data());
+    sim.transferAndPrepare();
+    sim.buildSystem();
+    auto resident = [&](uint32_t solves) {  // how many of them
+        uint32_t k = 0;
+        for (uint32_t i = 0; i < solves; ++i) {
+            const SolveStats st = sim.solve();
+            check(st.converged, "resident rest: converged");
+            k += st.residentRefinements > 0 ? 1u : 0u;
+        }
+        return k;
+    };
+    sim.setResidentPolls(0);
+    check(resident(1) == 0 && sim.residentGiveUps() == 1, "resident rest: first give-up");
+    check(resident(16) == 0 && sim.residentGiveUps() == 1, "resident rest: 16 solves");
+    check(resident(1) == 0 && sim.residentGiveUps() == 2, "resident rest: second give-up");
+    sim.setResidentPolls(ns::kResidentPolls);
+    check(resident(32) == 0 && sim.residentGiveUps() == 2, "resident rest: 32 solves");
+    check(resident(3) == 3 && sim.residentUsable(), "resident rest: resident again");
+    std::vector<double> q(sim.getArray("p", nullptr, 0));
+    sim.getArray("p", q.data(), q.size());
+    double d = 0.0, n = 0.0;
+    for (size_t i = 0; i < q.size(); ++i) d += (q[i] - p[1][i]) * (q[i] - p[1][i]), n += p[1][i] * p[1][i];
+    check(q.size() == p[1].size() && d <= 1e-8 * n, "resident rest: pressure");
+    sim.setResidentPolls(0);
+    check(resident(17) == 0 && sim.residentGiveUps() == 3, "resident rest: 16 solves again after a success");
+    sim.setResidentPolls(ns::kResidentPolls);
+    check(resident(1) == 1, "resident rest: resident after 16");
 }
 
 }  // namespace flip2

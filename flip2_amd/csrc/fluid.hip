@@ -599,10 +599,13 @@ SolveStats FluidSim::solveOnce(int prec, uint32_t capIn) {
     // only for caps that end a launch in a fraction of a second.
     const KernelTimer* timer = KernelTimer::current();
     const bool perIteration = capture_ || (timer && timer->asksFor("cg_"));
-    const ns::ResidentShape shape = !flex && !perIteration && residentOk_ && cap <= kResidentCap
-                                        ? ns::resident_shape(na, !jac)
-                                        : ns::ResidentShape{};
-    const bool resident = shape.groups > 0;
+    const ns::ResidentShape shape =
+        !flex && !perIteration && cap <= kResidentCap ? ns::resident_shape(na, !jac) : ns::ResidentShape{};
+    bool resident = shape.groups > 0;
+    if (resident && residentSkip_ > 0) {  // a wait of such a launch ran out a few solves ago
+        --residentSkip_;
+        resident = false;
+    }
     if (resident) {
         const size_t want = ns::resident_face_floats(na);
         if (faces_.size() < want) faces_.resizeAsync((uint32_t)ns::resident_face_floats(slotCapacity_), stream_);
@@ -656,10 +659,14 @@ SolveStats FluidSim::solveOnce(int prec, uint32_t capIn) {
             const double* r64 = refine == 0 ? b64_.devPtr() : r64_.devPtr();
             ResidentEnd end = residentRefinement(na, shape, !jac, r64, thr * thr, cap - total);
             if (end.failed) {  // x64 is not usable: solve again without it
-                residentOk_ = false;
+                // What held the chip may be gone in a moment or stay; a lost
+                // attempt takes ~0.2 s, so while it stays attempts get rarer.
+                residentRest_ = residentRest_ ? std::min(2u * residentRest_, kResidentMaxRest) : kResidentRest;
+                residentSkip_ = residentRest_ + 1u;  // this solve's second run takes one
                 ++residentGiveUps_;
                 return solveOnce(prec, capIn);
             }
+            residentRest_ = 0;
             total += end.iterations;
             rel = std::sqrt(std::max(end.rr, 0.0)) / st.bNorm;
             st.refinements = st.residentRefinements = refine + 1;

@@ -144,9 +144,12 @@ public:
     }
 
     // Reads that a wait between the resident PCG's workgroups may take before
-    // it is given up (the solve then runs again in the two-kernel form).
+    // it is given up (the solve then runs again in the two-kernel form, and so
+    // do the next solves: kResidentRest of them, twice as many after each
+    // further give-up in a row).
     void setResidentPolls(uint32_t polls) { residentPolls_ = polls; }
-    bool residentUsable() const { return residentOk_; }
+    bool residentUsable() const { return residentSkip_ == 0; }
+    static constexpr uint32_t kResidentRest = 16, kResidentMaxRest = 1024;
     // Solves of this simulation whose resident attempt was given up.
     uint32_t residentGiveUps() const { return residentGiveUps_; }
 
@@ -234,8 +237,9 @@ private:
     hipEvent_t histEvent_[2] = {nullptr, nullptr};
     double* pinnedHistory(size_t doubles);
     // The resident PCG (ns::launch_pcg_resident): its faces and published
-    // words, the number of its next sum, and whether it may be used (a wait
-    // between its workgroups ran out once: another process shares the GPU).
+    // words, the number of its next sum, and after a wait between its
+    // workgroups ran out (other work held the GPU's compute units) the solves
+    // left until it is tried again, residentRest_ at first.
     DeviceVec<float> faces_{dm_};
     DeviceVec<double> words_{dm_};
     struct ResidentEnd {
@@ -246,7 +250,7 @@ private:
     ResidentEnd residentRefinement(uint32_t na, const ns::ResidentShape& shape, bool mic, const double* r64,
                                    double thr2, uint32_t limit);
     uint32_t residentNumber_ = 0, residentPolls_ = ns::kResidentPolls, residentGiveUps_ = 0;
-    bool residentOk_ = true;
+    uint32_t residentSkip_ = 0, residentRest_ = 0;
     DeviceVec<uint32_t> total_{dm_};
     DeviceVec<uint8_t> ws_{dm_};
     uint32_t slotCapacity_ = 0;

@@ -351,7 +351,9 @@ int flip2_fluid_last_solve(flip2_fluid* f, flip2_solve_stats* stats);
  * one resident launch; two kernels per iteration serve larger systems,
  * iteration caps above 16384, residual capture, and solves whose resident
  * launch was given up (its workgroups wait for each other, and another
- * process held the GPU's compute units for ~0.2 s).  *resident_refinements:
+ * process held the GPU's compute units for ~0.2 s; the next 16 solves run the
+ * same way before it is tried again, twice as many after each further give-up
+ * in a row, up to 1024).  *resident_refinements:
  * refinements of the last solve that were one resident launch (0: the other
  * form, or the learned preconditioner).  *give_ups: solves of this simulation
  * so far whose resident attempt was given up.  Either may be NULL.  No
