@@ -12,6 +12,7 @@
 //
 //   flip2_tester [particles=20000] [cells=24] [seed=7]
 #include <algorithm>
+#include <chrono>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
@@ -338,6 +339,22 @@ void run_resident_fallback() {
     check(resident(17) == 0 && sim.residentGiveUps() == 3, "resident rest: 16 solves again after a success");
     sim.setResidentPolls(ns::kResidentPolls);
     check(resident(1) == 1, "resident rest: resident after 16");
+
+    // the solve's time includes the attempt that was given up: here it waits
+    // for 32 GB of fills queued before it, several times the solve's own time
+    void* big = nullptr;
+    const size_t bytes = (size_t)1 << 30;
+    check(hipMalloc(&big, bytes) == hipSuccess, "resident time: allocation");
+    sim.setResidentPolls(0);
+    for (int k = 0; k < 32; ++k)
+        check(hipMemsetAsync(big, k, bytes, sim.stream()) == hipSuccess, "resident time: fill");
+    const auto t0 = std::chrono::steady_clock::now();
+    const SolveStats st = sim.solve();
+    const double wall = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
+    check(hipFree(big) == hipSuccess, "resident time: free");
+    check(sim.residentGiveUps() == 4 && st.converged, "resident time: given up");
+    check(st.solveMs <= wall && st.solveMs >= 0.9 * wall, "resident time: the whole solve");
+    check(sim.lastSolve().solveMs == st.solveMs, "resident time: the last solve's");
 }
 
 }  // namespace flip2

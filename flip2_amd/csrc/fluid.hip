@@ -664,7 +664,12 @@ SolveStats FluidSim::solveOnce(int prec, uint32_t capIn) {
                 residentRest_ = residentRest_ ? std::min(2u * residentRest_, kResidentMaxRest) : kResidentRest;
                 residentSkip_ = residentRest_ + 1u;  // this solve's second run takes one
                 ++residentGiveUps_;
-                return solveOnce(prec, capIn);
+                const double lost =
+                    std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
+                st = solveOnce(prec, capIn);
+                st.solveMs += lost;
+                stats_ = st;
+                return st;
             }
             residentRest_ = 0;
             total += end.iterations;
