@@ -1,6 +1,6 @@
 // flip2_sort_pairs_u32_noalloc: the key/value radix sort of
-// flip2_sort_pairs_u32 with its workspace (digit histograms, digit offsets,
-// tile counters and the passes' look-back status words) in a fixed device
+// flip2_sort_pairs_u32 with its workspace (digit histograms, tile counters
+// and the passes' look-back status words) in a fixed device
 // array of this library instead of caller- or library-allocated memory, for
 // callers that cannot allocate (code under HIP graph capture, serving loops
 // that forbid hipMalloc).  Nothing here calls hipMalloc, hipFree or an

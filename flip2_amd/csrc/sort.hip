@@ -59,7 +59,7 @@ SortLayout sort_layout(uint32_t n, uint32_t beginBit, uint32_t endBit, int items
     L.passes = (endBit > beginBit) ? ceil_div(endBit - beginBit, 8) : 0;
     const uint32_t tiles = ceil_div(n ? n : 1, (uint32_t)items * kSortThreads);
     size_t off = 0;
-    L.histOff = off; off += (size_t)2 * kMaxPasses * kRadix * sizeof(uint32_t);
+    L.histOff = off; off += (size_t)kMaxPasses * kRadix * sizeof(uint32_t);
     L.counterOff = off; off += 256;
     L.statusOff = off; off += (size_t)L.passes * tiles * kRadix * sizeof(uint32_t);
     L.total = off + 256;

@@ -11,8 +11,10 @@ size_t sort_workspace_bytes(uint32_t n, uint32_t beginBit, uint32_t endBit);
 // (keysOut, valsOut).  valsIn == nullptr means values 0..n-1 (the sort
 // permutation).  keysAlt/valsAlt are ping-pong buffers (unused for a single
 // pass).  Inputs are not modified and must not alias any output buffer.
-// passEvents (optional, passes + 1 events): recorded after the histogram and
-// offset kernels and after each digit pass, for per-kernel timing.
+// passEvents (optional, passes + 1 events): recorded after the histogram kernel
+// and after each digit pass, for per-kernel timing.  A sort in one launch
+// records the first before it and the others after: all of its time lies
+// between the first two.
 // itemsPerThread: keys per lane of a digit-pass tile (4, 16, 24 or 32; 0 picks,
 // with a workspace of sort_workspace_bytes).
 void sort_pairs_u32(const uint32_t* keysIn, const uint32_t* valsIn, uint32_t* keysOut, uint32_t* valsOut,

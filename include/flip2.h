@@ -89,6 +89,9 @@ int flip2_scan_u32(const uint32_t* d_in, uint32_t* d_out, uint32_t n, int exclus
  * 0..n-1), which is the reference's reorderedGridIndices.  d_keys_alt /
  * d_vals_alt are ping-pong buffers of n elements (unused when one 8-bit pass
  * suffices).  Inputs are left unchanged and must not alias the outputs.
+ * flip2_sort_workspace_bytes is enough for n and every smaller count; from
+ * 4608 + 1024 * passes * ceil(n / 4096) bytes (passes: of 8 bits) a call is
+ * accepted, and below 2^18 keys is then slower than with the former.
  * Replaces cudaRadixSortUint (radixSortKernels.cu:85-123, radixSortKernels.hu:16-17)
  * and cudaSortParticlesByGridNode (particleToGridFunctions.cu:270-301). */
 size_t flip2_sort_workspace_bytes(uint32_t n, uint32_t begin_bit, uint32_t end_bit);

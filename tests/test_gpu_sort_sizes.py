@@ -1,8 +1,8 @@
 """The radix sort where its shape changes: the one-workgroup sort's two
 register sizes (4096 and 8192 keys), the 1024-, 4096- and 8192-key
 tiles and their remainders, every number of passes with whole and partial last
-digits, values and permutation, few distinct keys (stability), and a workspace
-shared by sorts of falling length.  Bit for bit against numpy's stable sort."""
+digits, values and permutation, few distinct keys (stability), a workspace
+shared by sorts of falling length, and the smallest workspace.  Bit for bit against numpy's stable sort."""
 import numpy as np
 import pytest
 
@@ -49,3 +49,29 @@ def test_workspace_covers_smaller_sorts(flip2):
         assert np.array_equal(bufs[1].to_array(np.uint32, m), ev)
     with pytest.raises(flip2.Flip2Error):
         flip2.check(L.flip2_sort_pairs_u32(dk.ptr, None, *(b.ptr for b in bufs), 5000, 0, 24, ws.ptr, 64, None))
+
+
+@pytest.mark.parametrize("n", [8193, 16385, 131073, 262143])
+def test_workspace_of_4096_key_tiles(flip2, n):
+    """The smallest workspace the header states: below it a call is refused,
+    with it sorts of the short tiles take the 4096-key ones."""
+    L = flip2.lib()
+    passes, end = 3, 24
+    least = 4608 + 1024 * passes * ((n + 4095) // 4096)
+    assert least < L.flip2_sort_workspace_bytes(n, 0, end)
+    rng = np.random.default_rng(n)
+    keys = rng.integers(0, 1 << end, n, dtype=np.uint64).astype(np.uint32)
+    dk, ws = flip2.DeviceBuffer.from_array(keys), flip2.DeviceBuffer(least)
+    bufs = [flip2.DeviceBuffer(4 * n) for _ in range(4)]
+    for ws_bytes in (least - 1, least):
+        args = (dk.ptr, None, *(b.ptr for b in bufs), n, 0, end, ws.ptr, ws_bytes, None)
+        if ws_bytes < least:
+            with pytest.raises(flip2.Flip2Error):
+                flip2.check(L.flip2_sort_pairs_u32(*args))
+            continue
+        for _ in range(2):  # the second call finds the first one's words in the workspace
+            flip2.check(L.flip2_sort_pairs_u32(*args))
+            flip2.synchronize()
+            ek, ev = _expect(keys, None, 0, end)
+            assert np.array_equal(bufs[0].to_array(np.uint32, n), ek)
+            assert np.array_equal(bufs[1].to_array(np.uint32, n), ev)
