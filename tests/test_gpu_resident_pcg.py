@@ -8,6 +8,8 @@ more than fits (both are then the two-kernel form).  Both solve to the same
 FP64 residual; with the same rounding of every vector update they take the
 same iterations up to the last few, and their pressures differ by the solver's
 tolerance times a factor for the operator's condition, far below 1e-4."""
+import threading
+
 import numpy as np
 import pytest
 
@@ -77,3 +79,41 @@ def test_resident_iteration_cap(flip2, prec):
         sim.close()
     assert got[0]["iterations"] == 7 and not got[0]["converged"]
     assert got[1]["converged"] and got[1]["iterations"] > 7
+
+
+def test_resident_on_threads(flip2):
+    """Simulations solving on threads of one process: their resident launches
+    take turns (each fits the chip by itself, not all together), every solve
+    stays resident, and each gives the iterations and pressure of the same
+    solve alone, bit for bit."""
+    sims, alone = [], []
+    for n, prec in ((64, "mic0"), (3100, "jacobi"), (900, "jacobi"), (2100, "mic0")):
+        grid, pos, vel = _bricks(n, n)
+        sim = flip2.FluidSim(pos[0].size, grid, preconditioner=prec)
+        sim.set_particles(*pos, *vel)
+        for stage in ("transfer_prepare", "system"):
+            sim.stage(stage)
+        s = sim.solve_with(prec)
+        assert s["converged"] and sim.solve_form()["resident_refinements"] == s["refinements"]
+        sims.append((sim, prec))
+        alone.append((s["iterations"], sim.get("p")))
+    got = [[] for _ in sims]
+
+    def work(k):
+        sim, prec = sims[k]
+        for _ in range(8):
+            s = sim.solve_with(prec)
+            got[k].append((s["iterations"], s["refinements"], sim.solve_form(), sim.get("p")))
+
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(len(sims))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for k, (iterations, p) in enumerate(alone):
+        assert len(got[k]) == 8
+        for its, refinements, form, q in got[k]:
+            assert its == iterations and np.array_equal(q, p)
+            assert form == {"resident_refinements": refinements, "give_ups": 0}
+    for sim, _ in sims:
+        sim.close()
