@@ -28,7 +28,7 @@ struct FluidConfig {
     int preconditioner = kPrecJacobi;
     double tolerance = 1e-6;       // ||b - A p||_2 / ||b||_2, FP64
     uint32_t maxIterations = 4000; // inner iterations over all refinements
-    uint32_t checkEvery = 8;       // iterations between host residual checks
+    uint32_t checkEvery = 8;       // two-kernel PCG: iterations between host residual checks
     float margin = 1e-3f;          // particles are kept this far (x h) inside the box
     // Learned preconditioner: fall back to Jacobi-PCG when flexible CG needs
     // more iterations than this (0: no fallback).

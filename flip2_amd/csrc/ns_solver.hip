@@ -1721,7 +1721,7 @@ __global__ void __launch_bounds__(256) g2p_advect_kernel(uint32_t n, float4* __r
 // entry ahead, so workgroups with light bricks take more of them.  With fewer
 // entries than half the workgroups, up to eight workgroups share an entry's
 // particles instead (a small scene waits for its fullest brick: 98 -> 13 us
-// at 48 bricks, 66 -> 37 at 160).
+// at 48 bricks, 66 -> 30 at 160).
 __global__ void __launch_bounds__(256)
 g2p_advect_brick_kernel(const uint32_t* __restrict__ list, const uint32_t* __restrict__ count,
                         uint32_t* __restrict__ counters, const uint32_t* __restrict__ brickStart, float4* __restrict__ rec, const float* __restrict__ U,

@@ -12,8 +12,12 @@
 // 9196 slots 54.5 -> 21.4 and 68.6 -> 22.9.
 // What bounds it: up to ~2000 slots the latency of the two sums (a write
 // and a read through memory each, ~1.5 us) and, with MIC(0), the chain of the
-// sweeps' 44 steps; above, the waves' instruction issue (~2400 per iteration
-// for four slots with MIC(0), half of them the sweeps).
+// sweeps' 44 steps; above, instruction issue beside the same waits: ~2500
+// instructions per wave and iteration for four slots with MIC(0), half of them
+// the sweeps.  2383 slots (one wave per SIMD): 4.2 of the 9.8 us at four clocks
+// each; 9196 slots (nine waves per CU, three on one of its SIMDs): 12.5 of the
+// 22.6 us, and waves wait for 65% of their time, among others for the registers
+// that do not fit (see below).
 //
 // Layout of large systems (pcg_resident_kernel; pcg_wide_kernel, one slot per
 // wave, has its own below).  A wave holds four slots, one per row of 16 lanes.  Lane 8 J + i of
@@ -26,7 +30,10 @@
 // The sweeps therefore run in registers (the two-kernel form exchanges every
 // plane through LDS and is bound by it: ~260 LDS instructions per slot).
 // Registers hold r, p, the factors and z / q; LDS holds e and the slot's six
-// faces of p (neighbours' cells).
+// faces of p (neighbours' cells).  That takes 218 registers (MIC(0)) and 241
+// (Jacobi), which up to eight waves per workgroup have; from nine on a lane has
+// 168, and 50 and 81 of them go to scratch memory and back in an iteration (25
+// reads and 8 writes per wave with MIC(0)).
 //
 // Per iteration: z = M^-1 r; the faces of z go out; sum r.z, r.r over the
 // grid; p = z + beta p for the own cells and, with the neighbours' faces of
@@ -808,6 +815,7 @@ ResidentKernel resident_kernel(bool mic, const ResidentShape& s) {
         return mic ? pcg_wide_kernel<1> : pcg_wide_kernel<0>;
     }
     // up to eight waves (two per SIMD) a lane may use 256 registers, above 168
+    // (which spills; the slots of nine to eleven waves have no other room)
     if (s.waves <= 8u) return mic ? pcg_resident_kernel<1, 8> : pcg_resident_kernel<0, 8>;
     return mic ? pcg_resident_kernel<1, kResidentMaxWaves> : pcg_resident_kernel<0, kResidentMaxWaves>;
 }
@@ -864,8 +872,9 @@ void launch_pcg_resident(const CgResident& c, const ResidentShape& shape, bool m
     // Per iteration without / with a pause (64 clocks each): 12 slots 4.66 ->
     // 4.58 us with 4 (5.25 with 18), 160 slots 4.70 -> 4.28 with 10 (4.69 with
     // 18), 960 slots 7.72 -> 5.47 with 18 (5.96 with 10), 9196 slots MIC(0)
-    // 25.0 -> 22.7 with 40 (24.2 with 18).
+    // 25.0 -> 22.6 with 36 (22.7 with 40, 24.2 with 18).
     k.pause = shape.groups <= 16u ? 4u : shape.groups <= 64u ? 10u : shape.waves <= 8u || shape.wide ? 18u : 36u;
+    // (a timer knows both layouts' kernels by this variable's name)
     FLIP2_KERNEL(pcg_resident_kernel, dim3(shape.groups), dim3(64 * shape.waves), lds, s, k);
     FLIP2_LAUNCH_CHECK();
 }

@@ -282,7 +282,9 @@ typedef struct flip2_fluid_config {
     int preconditioner;       /* FLIP2_PREC_* */
     double tolerance;         /* ||b - A p||_2 / ||b||_2 in FP64 */
     uint32_t max_iterations;  /* inner PCG iterations per solve */
-    uint32_t check_every;     /* iterations between residual checks */
+    uint32_t check_every;     /* iterations between the host's residual checks (the
+                                 result does not depend on it; a resident launch, see
+                                 flip2_fluid_solve_form, has none) */
     float margin;             /* particles kept margin*h inside the box */
 } flip2_fluid_config;
 
@@ -359,8 +361,10 @@ int flip2_fluid_last_solve(flip2_fluid* f, flip2_solve_stats* stats);
  * in a row, up to 1024).  *resident_refinements:
  * refinements of the last solve that were one resident launch (0: the other
  * form, or the learned preconditioner).  *give_ups: solves of this simulation
- * so far whose resident attempt was given up.  Either may be NULL.  No
- * counterpart in the reference. */
+ * so far whose resident attempt was given up.  Either may be NULL.  Resident
+ * launches of one process and device take turns: with simulations on several
+ * threads a solve waits for the others' launches.  No counterpart in the
+ * reference. */
 int flip2_fluid_solve_form(flip2_fluid* f, uint32_t* resident_refinements, uint32_t* give_ups);
 /* "U","V","W","U0","V0","W0","counts","cellStart","activeBricks","brickSlot",
  * "cellType","coef","b","p". */
@@ -369,7 +373,10 @@ int flip2_fluid_get_array(flip2_fluid* f, const char* name, void* host, size_t c
 /* Per-kernel timing with HIP events on the simulation's stream, for the
  * following flip2_fluid_step / _step_frame / _stage / _solve_with calls:
  * each launch of a kernel whose name is in the comma-separated list
- * `kernels` (NULL: every kernel) is bracketed by two events.  Launches
+ * `kernels` (NULL: every kernel) is bracketed by two events.  A resident
+ * solve's launches go by "pcg_resident_kernel"; a list with a name that begins
+ * with "cg_" (the two-kernel PCG's kernels) makes the timed solves take that
+ * form, also where an untimed one is resident.  Launches
  * captured into a HIP graph are not timed.  flip2_fluid_timing returns, for
  * timed kernel k (in name order), its name, the summed milliseconds and the
  * launch count (FLIP2_ERR_RANGE past the last one); enabling resets the
@@ -437,7 +444,7 @@ int flip2_fluid_set_unet(flip2_fluid* f, flip2_unet* net, uint32_t fallback_iter
 int flip2_fluid_set_flex_directions(flip2_fluid* f, uint32_t directions);
 /* Iterations (1..1024, default 1) between the host's residual checks in
  * flexible CG; the other solvers check every config.check_every
- * iterations.  No counterpart in the reference. */
+ * iterations where they check at all (see there).  No counterpart in the reference. */
 int flip2_fluid_set_flex_check_every(flip2_fluid* f, uint32_t iterations);
 /* The smoothing step around the learned correction (when the network has
  * a smoothing weight): FLIP2_SMOOTH_JACOBI (0) damped Jacobi with that
