@@ -18,7 +18,9 @@ Prints one JSON line.  value = particles x steps / wall seconds of the timed
 region (bracketed by device synchronisation).  roofline: the kernel with the
 largest share of an untimed profiled step; in the timed region only that
 kernel's launches are bracketed by HIP events on the simulation's stream,
-and its algorithmic bytes per launch / mean launch time give `achieved`.
+and its algorithmic bytes per launch / mean launch time give `achieved` (a
+resident PCG launch is bound by latency, not by that rate: its object also has
+the time per iteration).
 Extra keys: the same step on the 64^3 dam break (c1), the learned
 preconditioner against plain PCG on the 128^3 dam break with a sphere (c4,
 the committed network), and the 2^24-particle / 256^3 transfer microbench
@@ -248,9 +250,12 @@ def fluid_steps(cfg, steps, warmup, grid_c3=512, roofline=False):
         its = np.array([s["iterations"] for s in solves], np.float64)
         fcs = np.array([s["fluid_cells"] for s in solves], np.float64)
         fc = float((its * fcs).sum() / max(its.sum(), 1.0))  # fluid cells per solver launch
-        if dom == "pcg_resident_kernel":
+        resident = dom == "pcg_resident_kernel"
+        if resident:
             # one launch per refinement: the system in and the solution updated
-            # once, the bricks' six faces out and in at every iteration
+            # once, the bricks' six faces out and in at every iteration.  That
+            # rate is stated, but is not the kernel's limit: an iteration is two
+            # grid-wide sums and ~2500 instructions per wave of four bricks
             per_launch = float(its.sum()) / max(sum(s["refinements"] for s in solves), 1)
             bricks = float(np.mean([s["active_bricks"] for s in solves]))
             b = (2 + 4 + 8 + 16) * fc + per_launch * bricks * 2 * 6 * 64 * 4
@@ -258,17 +263,21 @@ def fluid_steps(cfg, steps, warmup, grid_c3=512, roofline=False):
             b = kernel_alg_bytes(dom, int(x.size), n ** 3, fc, jacobi=(prec == "jacobi"))
         achieved = b / (avg_ms * 1e-3) / 1e9 if b else None
         traffic = profiled_traffic(f"{cfg}_{n}", dom)
-        # launches of the dominant kernel in the timed steps, from the
-        # profiled step's launches per solver iteration
+        # launches of the dominant kernel in the timed steps: one per
+        # refinement, or from the profiled step's launches per solver iteration
         per_it = prof[dom][1] / max(prof_solve["iterations"], 1)
-        est_launches = per_it * float(its.sum())
+        est_launches = float(sum(s["refinements"] for s in solves)) if resident else per_it * float(its.sum())
         out["roofline"] = {
-            "bound": "hbm", "kernel": dom, "achieved": round(achieved, 1) if achieved else None,
+            "bound": "latency" if resident else "hbm", "kernel": dom,
+            "achieved": round(achieved, 1) if achieved else None,
             "peak": PEAK_HBM_GBPS, "unit": "GB/s", "frac": round(achieved / PEAK_HBM_GBPS, 4) if achieved else None,
             "traffic": traffic, "alg_bytes_per_launch": int(b) if b else None,
             "timed_launches": launches, "timing_sample_every": sample, "avg_launch_ms": round(avg_ms, 5),
             "share_of_timed_region": round(avg_ms * est_launches * 1e-3 / wall, 4),
             "fluid_cells_per_launch": int(fc)}
+        if resident:
+            out["roofline"].update(iterations_per_launch=round(per_launch, 1),
+                                   us_per_iteration=round(avg_ms * 1e3 / max(per_launch, 1.0), 2))
     sim.close()
     return out
 
