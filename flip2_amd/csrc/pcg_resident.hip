@@ -7,14 +7,14 @@
 // fit the chip's registers and LDS, so here an iteration moves only the
 // slots' faces (1.5 KB out and in per slot) and two grid-wide sums.  Per
 // iteration of a solve, two-kernel form -> this one: 160 slots Jacobi 14.5 ->
-// 4.3 us, MIC(0) 18.9 -> 6.7; 960 slots 18.5 -> 5.5 and 22.6 -> 7.6; 2383
-// slots 21.9 -> 6.9 and 31.7 -> 9.8; 4122 slots 33.6 -> 10.1 and 45.4 -> 13.7;
-// 9196 slots 54.5 -> 21.4 and 68.6 -> 22.9.
+// 4.3 us, MIC(0) 18.9 -> 6.7; 960 slots 18.5 -> 5.5 and 22.6 -> 7.7; 2383
+// slots 21.9 -> 6.9 and 31.7 -> 9.9; 4122 slots 33.6 -> 10.1 and 45.4 -> 13.7;
+// 9196 slots 54.5 -> 21.6 and 68.6 -> 22.6.
 // What bounds it: up to ~2000 slots the latency of the two sums (a write
 // and a read through memory each, ~1.5 us) and, with MIC(0), the chain of the
 // sweeps' 44 steps; above, instruction issue beside the same waits: ~2500
 // instructions per wave and iteration for four slots with MIC(0), half of them
-// the sweeps.  2383 slots (one wave per SIMD): 4.2 of the 9.8 us at four clocks
+// the sweeps.  2383 slots (one wave per SIMD): 4.2 of the 9.9 us at four clocks
 // each; 9196 slots (nine waves per CU, three on one of its SIMDs): 12.5 of the
 // 22.6 us, and waves wait for 65% of their time, among others for the registers
 // that do not fit (see below).
@@ -837,7 +837,7 @@ ResidentShape resident_shape(uint32_t na, bool mic) {
     // 7.3 -> 5.5 us, 1370 slots 7.3 -> 5.9 and MIC(0) 10.2 -> 9.2, 2508 slots
     // Jacobi 8.0 -> 7.4).  With MIC(0) only up to two waves per SIMD: beyond,
     // its sweeps, which keep four columns per lane busy in the other layout
-    // and one here, are bound by instruction issue (2383 slots 9.8 against
+    // and one here, are bound by instruction issue (2383 slots 9.9 against
     // 10.3 us).  At least four waves, one per SIMD: an iteration of a wave is
     // a chain of instructions, and fewer workgroups have fewer sums.
     s.wide = na <= (mic ? 8u : kWideMaxWaves) * most;
